@@ -87,6 +87,11 @@ extern "C" {
         gate_up: *const c_void, out: *mut c_void, num_rows: i32, intermediate_size: i32, dtype: i32,
         stream: *mut c_void,
     ) -> c_int;
+    /// New: rg_silu_and_mul on gate and up columns interleaved in blocks of 16.
+    pub fn rg_silu_and_mul_interleaved(
+        gate_up: *const c_void, out: *mut c_void, num_rows: i32, intermediate_size: i32, dtype: i32,
+        stream: *mut c_void,
+    ) -> c_int;
     /// Workspace size of the split-K form of v1 / v1_plus.
     pub fn rg_paged_attention_v1_workspace_bytes(
         batch_size: i32, num_heads: i32, num_kv_heads: i32, head_dim: i32, block_size: i32,

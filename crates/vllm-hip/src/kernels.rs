@@ -681,6 +681,19 @@ impl PagedAttentionKernels {
         status(ffi::rg_silu_and_mul(gate_up.as_ptr(), out.as_mut_ptr(), num_rows, intermediate_size, T::DTYPE,
                                     self.stream))
     }
+
+    /// launch_silu_and_mul on gate and up columns interleaved in blocks of 16 (the weight layout
+    /// of launch_linear_silu_mul).
+    pub unsafe fn launch_silu_and_mul_interleaved<T: KvElement>(
+        &self,
+        gate_up: &HipSlice<T>,
+        out: &mut HipSlice<T>,
+        num_rows: i32,
+        intermediate_size: i32,
+    ) -> CoreResult<()> {
+        status(ffi::rg_silu_and_mul_interleaved(gate_up.as_ptr(), out.as_mut_ptr(), num_rows, intermediate_size,
+                                                T::DTYPE, self.stream))
+    }
 }
 
 /// Host-side cos/sin table [max_position, head_dim] for RoPE (HF Llama convention).

@@ -197,6 +197,12 @@ int rg_rms_norm(const void* x, void* residual, const void* weight, void* out,
 int rg_silu_and_mul(const void* gate_up, void* out, int32_t num_rows,
                     int32_t intermediate_size, int32_t dtype, void* stream);
 
+/* rg_silu_and_mul on gate and up columns interleaved in blocks of 16 (columns 32j .. 32j+15:
+ * gate 16j .., columns 32j+16 .. 32j+31: up 16j ..), the order a GEMM with the weight layout of
+ * rg_linear_silu_mul leaves them in; intermediate_size a multiple of 16.  New entry. */
+int rg_silu_and_mul_interleaved(const void* gate_up, void* out, int32_t num_rows,
+                                int32_t intermediate_size, int32_t dtype, void* stream);
+
 /* Decode-step projection (candle's Linear::forward on a [tokens, in_features] activation,
  * crates/vllm-models/src/llama/architecture.rs:38-59,80-84, attention.rs:104-133):
  *   out[m, n] = round(sum_k x[m, k] * weight[n, k]),  m < num_rows, n < out_features,

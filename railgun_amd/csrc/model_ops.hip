@@ -113,9 +113,23 @@ __global__ __launch_bounds__(kRowThreads) void rms_norm_vec8_kernel(const uint4*
   }
 }
 
-// out[r, i] = round(round(silu(g)) * u) with g = gate_up[r, i], u = gate_up[r, inter + i]
+// out[r, i] = round(round(silu(g)) * u) with g the gate and u the up value of output i
 // (candle: silu(gate_proj(x)) * up_proj(x), each op rounded to the activation dtype).
 template <typename T>
+__device__ __forceinline__ float silu_mul_one(float g, float u) {
+  using E = elem<T>;
+  return E::to_f32(E::from_f32(g / (1.f + expf(-g)))) * u;
+}
+
+// Column of output i's gate value in a gate/up row, and the distance to its up value: gate
+// columns then up columns, or (IL) both interleaved in blocks of 16.
+template <bool IL>
+__device__ __forceinline__ int64_t gate_col(int i) { return IL ? 2 * (int64_t)i - (i & 15) : i; }
+template <bool IL>
+__device__ __forceinline__ int64_t up_step(int inter) { return IL ? 16 : inter; }
+
+// One output per thread: any width and alignment.
+template <typename T, bool IL>
 __global__ __launch_bounds__(kRowThreads) void silu_mul_kernel(const typename elem<T>::storage* __restrict__ gu,
                                                                typename elem<T>::storage* __restrict__ out,
                                                                int inter) {
@@ -123,10 +137,36 @@ __global__ __launch_bounds__(kRowThreads) void silu_mul_kernel(const typename el
   const int64_t r = blockIdx.y;
   const int i = blockIdx.x * kRowThreads + threadIdx.x;
   if (i >= inter) return;
-  const float g = E::to_f32(gu[r * 2 * inter + i]);
-  const float u = E::to_f32(gu[r * 2 * inter + inter + i]);
-  const float a = E::to_f32(E::from_f32(g / (1.f + expf(-g))));
-  out[r * inter + i] = E::from_f32(a * u);
+  const auto* row = gu + r * 2 * inter + gate_col<IL>(i);
+  out[r * inter + i] = E::from_f32(silu_mul_one<T>(E::to_f32(row[0]), E::to_f32(row[up_step<IL>(inter)])));
+}
+
+// 16-bit dtypes with inter % 8 == 0 and 16-byte aligned rows: 8 outputs per thread from one
+// 16-byte load of gate and one of up (a block of 16 interleaved columns holds two such runs).
+// Bound: memory, 6 bytes per output, with the exponential, the division and the roundings close
+// behind (rounding in software instead of pack2: 11.5 us).  At 860 rows of 8192 outputs (42 MB)
+// 13.5 us in the one-value form, 9.2 here (4.6 TB/s), and reading the interleaved columns where
+// the projection left them saves the pass that put them in order (18 us there).
+template <typename T, bool IL>
+__global__ __launch_bounds__(kRowThreads) void silu_mul_vec8_kernel(const uint16_t* __restrict__ gu,
+                                                                    uint16_t* __restrict__ out, int inter) {
+  using E = elem<T>;
+  const int64_t r = blockIdx.y;
+  const int i = 8 * (blockIdx.x * kRowThreads + threadIdx.x);
+  if (i >= inter) return;
+  const uint16_t* row = gu + r * 2 * inter + gate_col<IL>(i);
+  const uint4 g4 = *reinterpret_cast<const uint4*>(row);
+  const uint4 u4 = *reinterpret_cast<const uint4*>(row + up_step<IL>(inter));
+  const uint32_t gw[4] = {g4.x, g4.y, g4.z, g4.w}, uw[4] = {u4.x, u4.y, u4.z, u4.w};
+  uint32_t o[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float g0 = E::to_f32((uint16_t)(gw[k] & 0xffffu)), g1 = E::to_f32((uint16_t)(gw[k] >> 16));
+    const uint32_t a = pack2<T>(g0 / (1.f + expf(-g0)), g1 / (1.f + expf(-g1)));
+    o[k] = pack2<T>(E::to_f32((uint16_t)(a & 0xffffu)) * E::to_f32((uint16_t)(uw[k] & 0xffffu)),
+                    E::to_f32((uint16_t)(a >> 16)) * E::to_f32((uint16_t)(uw[k] >> 16)));
+  }
+  *reinterpret_cast<uint4*>(out + r * inter + i) = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -168,23 +208,50 @@ extern "C" int rg_rms_norm(const void* x, void* residual, const void* weight, vo
   });
 }
 
-extern "C" int rg_silu_and_mul(const void* gate_up, void* out, int32_t num_rows, int32_t intermediate_size,
-                               int32_t dtype, void* stream) {
-  const char* op = "silu_and_mul";
+namespace rg {
+namespace {
+template <bool IL>
+int silu_and_mul_entry(const char* op, const void* gate_up, void* out, int32_t num_rows, int32_t intermediate_size,
+                       int32_t dtype, void* stream) {
   if (dtype_bytes(dtype) == 0) return fail(RG_ERR_NOT_SUPPORTED, "%s: unknown dtype %d", op, dtype);
   if (num_rows < 0 || intermediate_size <= 0 || num_rows > 65535) {
     return fail(RG_ERR_INVALID_ARGUMENT, "%s: need 0 <= num_rows <= 65535 and intermediate_size > 0 (got %d, %d)",
                 op, num_rows, intermediate_size);
   }
+  if (IL && intermediate_size % 16 != 0) {
+    return fail(RG_ERR_NOT_SUPPORTED, "%s: intermediate_size must be a multiple of 16 (got %d)", op,
+                intermediate_size);
+  }
   if (num_rows == 0) return ok();
   if (!gate_up || !out) return fail(RG_ERR_INVALID_ARGUMENT, "%s: null pointer argument", op);
   hipStream_t s = as_stream(stream);
-  const dim3 grid((unsigned)ceil_div(intermediate_size, kRowThreads), (unsigned)num_rows);
+  const bool vec = dtype != RG_DTYPE_F32 && intermediate_size % 8 == 0 && aligned16(gate_up) && aligned16(out);
+  const dim3 grid((unsigned)ceil_div(intermediate_size, (vec ? 8 : 1) * kRowThreads), (unsigned)num_rows);
   return dispatch_dtype(dtype, [&](auto tag) {
     using T = decltype(tag);
     using S = typename elem<T>::storage;
-    hipLaunchKernelGGL(silu_mul_kernel<T>, grid, dim3(kRowThreads), 0, s, static_cast<const S*>(gate_up),
+    if constexpr (!std::is_same_v<T, f32_t>) {
+      if (vec) {
+        hipLaunchKernelGGL((silu_mul_vec8_kernel<T, IL>), grid, dim3(kRowThreads), 0, s,
+                           static_cast<const uint16_t*>(gate_up), static_cast<uint16_t*>(out), intermediate_size);
+        return check_launch(op);
+      }
+    }
+    hipLaunchKernelGGL((silu_mul_kernel<T, IL>), grid, dim3(kRowThreads), 0, s, static_cast<const S*>(gate_up),
                        static_cast<S*>(out), intermediate_size);
     return check_launch(op);
   });
+}
+}  // namespace
+}  // namespace rg
+
+extern "C" int rg_silu_and_mul(const void* gate_up, void* out, int32_t num_rows, int32_t intermediate_size,
+                               int32_t dtype, void* stream) {
+  return silu_and_mul_entry<false>("silu_and_mul", gate_up, out, num_rows, intermediate_size, dtype, stream);
+}
+
+extern "C" int rg_silu_and_mul_interleaved(const void* gate_up, void* out, int32_t num_rows,
+                                           int32_t intermediate_size, int32_t dtype, void* stream) {
+  return silu_and_mul_entry<true>("silu_and_mul_interleaved", gate_up, out, num_rows, intermediate_size, dtype,
+                                  stream);
 }

@@ -42,9 +42,9 @@ import torch.nn.functional as F
 
 from .batch import StepBatch
 from .kv_pool import GpuBlockPool
-from .ops import (LINEAR_MAX_ROWS, PagedAttentionKernels, deinterleave_gate_up, interleave_gate_up, linear,
-                  linear_residual, linear_silu_mul, linear_workspace_bytes, rms_norm, rope_cos_sin_table,
-                  silu_and_mul)
+from .ops import (LINEAR_MAX_ROWS, PagedAttentionKernels, interleave_gate_up, linear, linear_residual,
+                  linear_silu_mul, linear_workspace_bytes, rms_norm, rope_cos_sin_table, silu_and_mul,
+                  silu_and_mul_interleaved)
 
 log = logging.getLogger(__name__)
 
@@ -351,9 +351,10 @@ class RailgunLlama:
             self._mlp_act_separate(layer, h, act)
 
     def _mlp_act_separate(self, layer: int, h: torch.Tensor, act: torch.Tensor) -> None:
-        """The gate/up projection, then rg_silu_and_mul over [gate | up] columns."""
-        y = self._linear(h, "w_gate_up", layer)
-        silu_and_mul(deinterleave_gate_up(y) if self.w.layers[layer].gate_up_interleaved else y, act)
+        """The gate/up projection, then rg_silu_and_mul over its columns in the order the weight
+        is held in."""
+        gate = silu_and_mul_interleaved if self.w.layers[layer].gate_up_interleaved else silu_and_mul
+        gate(self._linear(h, "w_gate_up", layer), act)
 
     def _qkv_rope_cache(self, layer: int, h: torch.Tensor, q: torch.Tensor, st: DeviceStep) -> None:
         """q/k/v = h @ wqkv^T, RoPE on q and k, k and v into the paged cache: fused in the

@@ -478,16 +478,25 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, eps: floa
                                      rows, hidden, dtype_code(x), _stream(x)))
 
 
-def silu_and_mul(gate_up: torch.Tensor, out: torch.Tensor) -> None:
-    """out [rows, I] = silu(gate_up[:, :I]) * gate_up[:, I:] (rg_silu_and_mul)."""
+def _silu_and_mul(fn, gate_up: torch.Tensor, out: torch.Tensor) -> None:
     _require_cuda(gate_up, out)
     if not gate_up.is_contiguous() or not out.is_contiguous() or gate_up.dtype != out.dtype:
         raise RailgunError(_lib.RG_ERR_INVALID_ARGUMENT, "silu_and_mul: tensors must be contiguous, one dtype")
     rows, inter = int(out.shape[0]), int(out.shape[-1])
     if tuple(gate_up.shape) != (rows, 2 * inter):
         raise RailgunError(_lib.RG_ERR_INVALID_ARGUMENT, "silu_and_mul: gate_up must be [rows, 2 * I]")
-    check(load_library().rg_silu_and_mul(gate_up.data_ptr(), out.data_ptr(), rows, inter, dtype_code(out),
-                                         _stream(out)))
+    check(fn(gate_up.data_ptr(), out.data_ptr(), rows, inter, dtype_code(out), _stream(out)))
+
+
+def silu_and_mul(gate_up: torch.Tensor, out: torch.Tensor) -> None:
+    """out [rows, I] = silu(gate_up[:, :I]) * gate_up[:, I:] (rg_silu_and_mul)."""
+    _silu_and_mul(load_library().rg_silu_and_mul, gate_up, out)
+
+
+def silu_and_mul_interleaved(gate_up: torch.Tensor, out: torch.Tensor) -> None:
+    """silu_and_mul(deinterleave_gate_up(gate_up), out) without the copy: gate_up [rows, 2 I] with
+    its columns interleaved in blocks of 16 (rg_silu_and_mul_interleaved; I a multiple of 16)."""
+    _silu_and_mul(load_library().rg_silu_and_mul_interleaved, gate_up, out)
 
 
 # Rows up to which rg_linear serves a projection (decode batches); larger ones go to hipBLASLt.
@@ -610,4 +619,4 @@ def linear_residual(x: torch.Tensor, weight: torch.Tensor, residual: torch.Tenso
 __all__ = ["LINEAR_MAX_ROWS", "PagedAttentionKernels", "PagedAttentionOp", "RailgunError", "cache_geometry",
            "deinterleave_gate_up", "dtype_code", "interleave_gate_up", "linear", "linear_residual",
            "linear_silu_mul", "linear_workspace_bytes", "rms_norm", "rope_cos_sin_table", "silu_and_mul",
-           "V1_MAX_CONTEXT", "V2_PARTITION_SIZE"]
+           "silu_and_mul_interleaved", "V1_MAX_CONTEXT", "V2_PARTITION_SIZE"]

@@ -24,7 +24,7 @@ from oracle import llama_ref
 from railgun_amd.batch import DecodeSlot, PrefillChunk, pack_step
 from railgun_amd.kv_pool import GpuBlockPool
 from railgun_amd.llama import DeviceStep, LlamaConfig, LlamaWeights, RailgunLlama
-from railgun_amd.ops import deinterleave_gate_up, rms_norm, rope_cos_sin_table, silu_and_mul
+from railgun_amd.ops import deinterleave_gate_up, rms_norm, rope_cos_sin_table, silu_and_mul, silu_and_mul_interleaved
 
 pytestmark = pytest.mark.gpu
 transformers = pytest.importorskip("transformers")
@@ -66,6 +66,26 @@ def test_silu_and_mul(device, inter):
     a = _bf16_round(torch.nn.functional.silu(gu[:, :inter].float()))
     want = a * gu[:, inter:].float()
     torch.testing.assert_close(out.cpu().float(), want, atol=1e-6, rtol=2 ** -7)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,inter,skip", [(1, 16, 0), (9, 2048, 0), (3, 2064, 0), (257, 4112, 0), (5, 48, 4)])
+def test_silu_and_mul_interleaved(device, dt, rows, inter, skip):
+    """Bit-equal to rg_silu_and_mul on the de-interleaved columns: one block, the edge of a
+    workgroup's columns and past it, and an unaligned buffer (the one-value form)."""
+    g = torch.Generator().manual_seed(rows * inter)
+    flat = (3 * torch.randn(rows * 2 * inter + skip, generator=g)).to(dt).to(device)
+    gu = flat[skip:].view(rows, 2 * inter)
+    got, want = torch.empty(rows, inter, dtype=dt, device=device), torch.empty(rows, inter, dtype=dt, device=device)
+    silu_and_mul_interleaved(gu, got)
+    silu_and_mul(deinterleave_gate_up(gu), want)
+    assert torch.equal(got, want)
+    gate, up = deinterleave_gate_up(gu.cpu()).float().chunk(2, -1)
+    a = torch.nn.functional.silu(gate).to(dt).float()
+    # 16 bits: silu may round the other way (one ulp, at most eps) and the product is rounded (half
+    # an ulp): 2 eps.  fp32: exp within 2 ulp on either side, a sum, a division and a product: 8 eps.
+    eps = torch.finfo(dt).eps
+    torch.testing.assert_close(got.cpu().float(), a * up, atol=1e-6, rtol=(8 if dt == torch.float32 else 2) * eps)
 
 
 @pytest.mark.parametrize("D,H,Hkv", [(64, 32, 8), (128, 8, 2)])
