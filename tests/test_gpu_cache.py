@@ -126,3 +126,27 @@ def test_rope_reshape_and_cache_bit_exact(device, kernels, which):
     np.testing.assert_array_equal(from_dev(dk, dt).view(np.uint8), k_before.view(np.uint8))
     np.testing.assert_array_equal(from_dev(dkc, dt).view(np.uint8), kc.view(np.uint8))
     np.testing.assert_array_equal(from_dev(dvc, dt).view(np.uint8), vc.view(np.uint8))
+
+
+@pytest.mark.parametrize("D,skip", [(8, 0), (16, 0), (64, 0), (128, 0), (256, 0), (24, 0), (64, 1)])
+def test_rope_reshape_and_cache_f32_bit_exact(device, kernels, D, skip):
+    """fp32: the 16-byte kernel from one chunk per half row to 32, a width whose chunks do not
+    divide the workgroup (24) and a q one element off its alignment (both the one-pair form)."""
+    rng = np.random.default_rng(D + skip)
+    T, H, hkv, bs, nb, dt = 21, 6, 2, 16, 5, "f32"
+    q, k, v = normal(rng, (T, H, D), dt), normal(rng, (T, hkv, D), dt), normal(rng, (T, hkv, D), dt)
+    pool = normal(rng, (nb, 2, hkv, bs, D), dt)
+    pos = rng.integers(0, 300, size=T).astype(np.int32)
+    slots = _slots(rng, T, nb, bs)
+    table = rope_cos_sin_table(300, D, 500000.0)
+    flat = torch.zeros(q.size + skip, device=device)
+    dq = flat[skip:].view(T, H, D).copy_(to_dev(q, dt, device))
+    dpool = to_dev(pool, dt, device)
+    kernels.launch_rope_reshape_and_cache(dq, to_dev(k, dt, device), to_dev(v, dt, device), dpool[:, 0], dpool[:, 1],
+                                          table.to(device), i32(pos, device), i32(slots, device), H, hkv, D, bs, T)
+    torch.cuda.synchronize()
+    orc.rope(q, table.numpy(), pos, dt)
+    orc.rope(k, table.numpy(), pos, dt)
+    orc.reshape_and_cache(k, v, pool[:, 0], pool[:, 1], slots, dt, bs, kv_block_stride=2 * hkv * bs * D)
+    np.testing.assert_array_equal(from_dev(dq, dt).view(np.uint8), q.view(np.uint8))
+    np.testing.assert_array_equal(from_dev(dpool, dt).view(np.uint8), pool.view(np.uint8))
