@@ -1049,8 +1049,19 @@ __global__ __launch_bounds__(kPThreads, pf_wg_per_cu<D>()) void prefill_mfma_ker
 // the units with most keys start first and the short ones fill in behind them, and with the head
 // group as the fastest dimension a multiple of 8 groups keeps each kv-head's K/V on one die.  The
 // order before it, units ascending with the head group slowest, started the longest units last:
-// 5 prompts of 171 to 964 tokens at 32 / 8 heads of 64 took 177 us, 146 now.  The 32-key K and V tiles reach LDS by direct global -> LDS
-// copies into two buffers, tile kt + 1 in flight while tile kt computes.
+// 5 prompts of 171 to 964 tokens at 32 / 8 heads of 64 took 177 us, 146
+// with the loop of that time.
+//
+//  * Bound: the fp32 MFMAs, 64 cycles each, 2 x D / 2 of them per tile.  The 32-key K and V tiles
+//    reach LDS by direct global -> LDS copies into two buffers each, K a tile further ahead than
+//    V, and iteration kt runs the QK MFMAs of tile kt + 1 with the softmax of tile kt between
+//    them, both operands read from LDS a few steps ahead of their MFMA, so that a wave keeps its
+//    SIMD's matrix core busy by itself: the last units of a call run one or two to a CU.  Without
+//    that (QK, softmax, PV in turn, operands read as they were used, a table read in front of
+//    every copy) the 5 prompts above took 146 us, 113 with it (75 TFLOP/s, 49 % of what a large
+//    fp32 product reaches here); 12 prompts of 128 to 2,048 tokens at head_dim 128 2,158 -> 1,749
+//    us a call with the cache write, 6 of up to 700 behind up to 500 cached at head_dim 256 529 ->
+//    304.  The arithmetic and its order are unchanged.
 //
 //  * Scores transposed, S^T = K Q^T: lane (row l % 32, half h = l / 32) provides K[key l % 32]
 //    and Q[query l % 32] at the d of MFMA k-index h; inside a pair of steps the d order is
@@ -1112,30 +1123,42 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
     const int nkeys = __builtin_amdgcn_readfirstlane(max(0, min(min(ctx, key_cap), first_v + last_row + 1)));
     const int ntiles = (nkeys + kPT - 1) / kPT;
 
-    // Copies of tile kt into buffer kt % 2: copy i of wave w moves LDS pieces
-    // 64 (w PER + i) + lane; keys past the unit's last read the last one (masked below).  The
-    // block-table reads come first, so that no wait for one of them falls between copies.
-    auto issue = [&](int kt) __attribute__((always_inline)) {
+    // Copy i of wave w moves LDS pieces 64 (w PER + i) + lane of an operand's tile; keys past the
+    // unit's last read the last one (masked below).  Lane l holds the cache offset of key l % 32
+    // of a tile: its block number is loaded two iterations before its K copy (table_entry) and
+    // turned into the offset (row_offset) when that copy goes out, so that no copy waits for a
+    // table read; the V copies fetch the offsets of their rows from those lanes.
+    const int kl = lane & 31;
+    int blk = 0, in_blk = 0;
+    auto table_entry = [&](int kt) __attribute__((always_inline)) {
+      const int kk = min(kt * kPT + kl, nkeys - 1);
+      const int b = kk / bs;
+      in_blk = kk - b * bs;
+      blk = bt[b];
+    };
+    auto row_offset = [&]() __attribute__((always_inline)) {
+      return (int64_t)blk * a.kv_stride + ((int64_t)kvh * bs + in_blk) * D;
+    };
+    auto issue_k = [&](int kt, int64_t roff) __attribute__((always_inline)) {
       const uint32_t off = (uint32_t)((kt & 1) * TILE * 4);
-      int64_t ksrc[PER], vsrc[PER];
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
+      for (int i = 0; i < PER; ++i) {  // K image [d / 4][key][4]: piece pc is key pc % 32, d / 4 = pc / 32
         const int pc = 64 * (w * PER + i) + lane;
-        const int kk = min(kt * kPT + pc % kPT, nkeys - 1);   // K image [d / 4][key][4]
-        ksrc[i] = (int64_t)bt[kk / bs] * a.kv_stride + ((int64_t)kvh * bs + kk % bs) * D + 4 * (pc / kPT);
-        const int vk = min(kt * kPT + pc / NC, nkeys - 1);     // V image row-major
-        vsrc[i] = (int64_t)bt[vk / bs] * a.kv_stride + ((int64_t)kvh * bs + vk % bs) * D + 4 * (pc % NC);
+        lds_dma16(kc + roff + 4 * (pc / kPT), k_base + off + (uint32_t)(64 * (w * PER + i)) * 16);
       }
-      // Every address is formed (the compiler's waits for the table reads placed) before the
-      // first copy: a wait it placed after a copy would wait for that copy too.
+    };
+    auto issue_v = [&](int kt, int64_t roff) __attribute__((always_inline)) {
+      const uint32_t off = (uint32_t)((kt & 1) * TILE * 4);
+      int64_t src[PER];
 #pragma unroll
-      for (int i = 0; i < PER; ++i) asm volatile("" ::"v"(ksrc[i]), "v"(vsrc[i]));
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const uint32_t dst = off + (uint32_t)(64 * (w * PER + i)) * 16;
-        lds_dma16(kc + ksrc[i], k_base + dst);
-        lds_dma16(vc + vsrc[i], v_base + dst);
+      for (int i = 0; i < PER; ++i) {  // V image row-major
+        const int pc = 64 * (w * PER + i) + lane;
+        const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)roff, pc / NC);
+        const int hi = __shfl((int)(roff >> 32), pc / NC);
+        src[i] = ((int64_t)hi << 32 | lo) + 4 * (pc % NC);
       }
+#pragma unroll
+      for (int i = 0; i < PER; ++i) lds_dma16(vc + src[i], v_base + off + (uint32_t)(64 * (w * PER + i)) * 16);
     };
 
     float qr[NC][2];
@@ -1162,63 +1185,156 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
     const int wrow0 = unit * UR + sub * kPT;
     const int wlast = first + min(wrow0 + kPT, L) - 1;
     const int kfull = !kSkip ? ntiles : wrow0 < L && wlast >= 0 ? min(ntiles, wlast / kPT + 1) : 0;
-    if (ntiles > 0) issue(0);
-    for (int kt = 0; kt < kfull; ++kt) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies of tile kt
-      tile_barrier();                                   // ... and every wave's
-      if (kt + 1 < ntiles) issue(kt + 1);               // the buffer tile kt - 1 used
-      const float* kt_lds = k_lds[kt & 1];
-      const float* vt_lds = v_lds[kt & 1];
+    // Tiles below kclear need no mask: every key at or before the wave's first row and present.
+    const int kclear = min(max(first + wrow0 + 1, 0), nkeys) / kPT;
 
-      // S^T = K Q^T over d: steps (c, e).
+    // S^T = K Q^T of tile kt over d: steps (c, e), the K operands read kAhead steps c ahead of
+    // their MFMAs; between(c) is the work that rides along with step c.
+    constexpr int kAhead = 4;
+    auto scores = [&](int kt, auto between) __attribute__((always_inline)) {
+      const float* kt_lds = k_lds[kt & 1] + qi * 4 + 2 * h;
       f32x16 st = f32x16{};
+      float2 kv[kAhead];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const float2 kv = *reinterpret_cast<const float2*>(kt_lds + (c * kPT + qi) * 4 + 2 * h);
-        st = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qr[c][0], st, 0, 0, 0);
-        st = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qr[c][1], st, 0, 0, 0);
-      }
-      // Mask, tile maximum, online softmax (log2 units).
-      float mx = -INFINITY;
+      for (int c = 0; c < kAhead; ++c) kv[c] = *reinterpret_cast<const float2*>(kt_lds + c * kPT * 4);
+      [&]<int... C>(std::integer_sequence<int, C...>) __attribute__((always_inline)) {
+        ([&] __attribute__((always_inline)) {
+          const float2 k2 = kv[C % kAhead];
+          if constexpr (C + kAhead < NC) {
+            kv[C % kAhead] = *reinterpret_cast<const float2*>(kt_lds + (C + kAhead) * kPT * 4);
+          }
+          st = __builtin_amdgcn_mfma_f32_32x32x2f32(k2.x, qr[C][0], st, 0, 0, 0);
+          between(std::integral_constant<int, C>{});
+          st = __builtin_amdgcn_mfma_f32_32x32x2f32(k2.y, qr[C][1], st, 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }(), ...);
+      }(std::make_integer_sequence<int, NC>{});
+      return st;
+    };
+    // Keys of tile kt that a row does not attend to, on the tiles that hold any.
+    auto mask = [&](f32x16& st, int kt) __attribute__((always_inline)) {
+      if (kt < kclear) return;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int key = kt * kPT + 8 * j + 4 * h + r;
           if (!row_ok || key > qpos || key >= nkeys) st[4 * j + r] = -INFINITY;
-          mx = fmaxf(mx, st[4 * j + r]);
         }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float mn = fmaxf(m, mx);
-      const float alpha = mn == -INFINITY ? 1.f : exp2f(m - mn);
-      float ps = 0.f;
+    };
+    // Online softmax (log2 units) of scores st, which become probabilities, in the parts 0 .. 11
+    // that ride along with the next tile's QK steps; rescale then applies the new maximum to o.
+    float mx = 0.f, mref = 0.f, alpha = 0.f, ps = 0.f;
+    bool moved = false;
+    auto softmax_part = [&](f32x16& st, auto part) __attribute__((always_inline)) {
+      constexpr int P = decltype(part)::value;
+      if constexpr (P == 0) {
+        mx = st[0];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float pe = mn == -INFINITY ? 0.f : exp2f(st[e] - mn);
-        st[e] = pe;
-        ps += pe;
+        for (int e = 1; e < 16; ++e) mx = fmaxf(mx, st[e]);
+      } else if constexpr (P == 1) {
+        ps = __shfl_xor(mx, 32, 64);
+      } else if constexpr (P == 3) {
+        const float mn = fmaxf(m, fmaxf(mx, ps));
+        // A row without a key yet keeps its maximum of -inf: 0 in its place gives exponents of
+        // -inf - 0, probabilities 0.
+        mref = mn == -INFINITY ? 0.f : mn;
+        alpha = __builtin_amdgcn_exp2f(m - mref);
+        moved = __ballot(m != mn) != 0;  // else every alpha that matters is exactly 1
+        m = mn;
+        ps = 0.f;
+      } else if constexpr (P >= 4 && P < 12) {
+#pragma unroll
+        for (int e = 2 * (P - 4); e < 2 * (P - 4) + 2; ++e) {
+          float pe = __builtin_amdgcn_exp2f(st[e] - mref);
+          ps += pe;
+          asm volatile("" : "+v"(pe));  // formed here, not behind the branch of rescale
+          st[e] = pe;
+        }
+        if constexpr (P == 11) lsum = lsum * alpha + ps;
       }
-      lsum = lsum * alpha + ps;
-      m = mn;
+    };
+    auto rescale = [&]() __attribute__((always_inline)) {
+      if (moved) {
 #pragma unroll
-      for (int b = 0; b < NDB; ++b) o[b] *= alpha;
-      // O^T += V^T P^T over the tile's keys: steps (j, r).
+        for (int b = 0; b < NDB; ++b) o[b] *= alpha;
+      }
+    };
+    // O^T += V^T P^T over tile kt's keys: steps i = (j, r), the V operands kAhead steps ahead.
+    auto accumulate = [&](const f32x16& st, int kt) __attribute__((always_inline)) {
+      const float* vt_lds = v_lds[kt & 1] + 4 * h * D + qi;
+      auto vrow = [&](int i) { return vt_lds + (8 * (i / 4) + i % 4) * D; };
+      float va[kAhead][NDB];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int i = 0; i < kAhead; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float* vrow = vt_lds + (8 * j + 4 * h + r) * D + qi;
+        for (int b = 0; b < NDB; ++b) va[i][b] = vrow(i)[32 * b];
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int b = 0; b < NDB; ++b) {
-            o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * b], st[4 * j + r], o[b], 0, 0, 0);
-          }
+      for (int i = 0; i < 16; ++i) {
+        float v[NDB];
+#pragma unroll
+        for (int b = 0; b < NDB; ++b) v[b] = va[i % kAhead][b];
+        if (i + kAhead < 16) {
+#pragma unroll
+          for (int b = 0; b < NDB; ++b) va[i % kAhead][b] = vrow(i + kAhead)[32 * b];
         }
-    }
-    if constexpr (kSkip) {
-      for (int kt = kfull; kt < ntiles; ++kt) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        tile_barrier();
-        if (kt + 1 < ntiles) issue(kt + 1);
+#pragma unroll
+        for (int b = 0; b < NDB; ++b) {
+          o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[b], st[i], o[b], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+
+    // Iteration kt waits for K(kt + 1) and V(kt), sends out K(kt + 2) and V(kt + 1) into the
+    // buffers that K(kt) and V(kt - 1) have left, and runs the QK MFMAs of tile kt + 1 under the
+    // softmax of tile kt: a wave alone on its SIMD then keeps the matrix core busy through the
+    // softmax.
+    if (ntiles > 0) {
+      int64_t roff1;
+      table_entry(0);
+      {
+        const int64_t roff0 = row_offset();
+        table_entry(1);
+        issue_k(0, roff0);
+        issue_v(0, roff0);
+      }
+      roff1 = row_offset();
+      table_entry(2);
+      if (ntiles > 1) issue_k(1, roff1);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      tile_barrier();
+      f32x16 st = f32x16{};
+      if (kfull > 0) st = scores(0, [](auto) {});
+      auto copies = [&](int kt) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // this wave's copies (and LDS reads)
+        tile_barrier();                                              // ... and every wave's
+        const int64_t roff2 = row_offset();
+        table_entry(kt + 3);
+        if (kt + 2 < ntiles) issue_k(kt + 2, roff2);
+        if (kt + 1 < ntiles) issue_v(kt + 1, roff1);
+        roff1 = roff2;
+      };
+      for (int kt = 0; kt < kfull - 1; ++kt) {
+        copies(kt);
+        mask(st, kt);
+        const f32x16 nx = scores(kt + 1, [&](auto c) __attribute__((always_inline)) { softmax_part(st, c); });
+        rescale();
+        accumulate(st, kt);
+        st = nx;
+      }
+      if (kfull > 0) {
+        copies(kfull - 1);
+        mask(st, kfull - 1);
+        [&]<int... P>(std::integer_sequence<int, P...>) __attribute__((always_inline)) {
+          (softmax_part(st, std::integral_constant<int, P>{}), ...);
+        }(std::make_integer_sequence<int, 12>{});
+        rescale();
+        accumulate(st, kfull - 1);
+      }
+      if constexpr (kSkip) {
+        for (int kt = kfull; kt < ntiles; ++kt) copies(kt);
       }
     }
     // The two halves of a query's row sum; rows without keys (or past the sequence) give 0.
