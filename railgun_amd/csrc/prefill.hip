@@ -1039,18 +1039,94 @@ __global__ __launch_bounds__(kPThreads, pf_wg_per_cu<D>()) void prefill_mfma_ker
   }  // units of this workgroup
 }
 
+// The i-th of a batch's units of UR rows, most keys first: unit u of a sequence whose first new row
+// sits at position `first` has the work key floor(max(first, 0) / UR) + u, so a key occurs at most
+// once per sequence, and the units of at least a given key are counted with one sum over the
+// sequences (one per lane, 64 at a time): a binary search over the keys, then the sequences of the
+// key found in order.  Returned wave-uniform; seq = -1 past the last unit.
+// With cols > 0 the first 2 cols units start at once and workgroups i and i + cols share a CU: the
+// second cols units are dealt in reverse, so that the longest of them go with the shortest of the
+// first.
+struct UnitAt { int seq, unit, row0, rows, ctx; };
+__device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t* ctx_lens, int num_seqs, int UR,
+                                               int i, int cols) {
+  const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+  int c_loaded = -1, row0 = 0, rows = 0, ctx = 0, base = 0, n = 0;
+  auto load = [&](int c) {  // the sequences of chunk c, one per lane
+    if (c == c_loaded) return;
+    c_loaded = c;
+    const int s = c * 64 + lane;
+    row0 = rows = ctx = base = n = 0;
+    if (s < num_seqs) {
+      row0 = cu[s];
+      rows = cu[s + 1] - row0;
+      ctx = ctx_lens[s];
+      n = rows > 0 ? (rows + UR - 1) / UR : 0;
+      base = max(ctx - rows, 0) / UR;
+    }
+  };
+  const int chunks = (num_seqs + 63) / 64;
+  auto sum = [](int v) { return __builtin_amdgcn_readlane(wave_prefix_sum(v), 63); };
+  auto count = [&](int k) {  // units whose key is at least k
+    int t = 0;
+    for (int c = 0; c < chunks; ++c) {
+      load(c);
+      t += sum(min(max(base + n - k, 0), n));
+    }
+    return t;
+  };
+  UnitAt u{-1, 0, 0, 0, 0};
+  const int total = count(0);
+  if (i >= cols && i < 2 * cols) i = 3 * cols - 1 - i;
+  if (i >= total) return u;
+  int lo = 0, hi = 0;
+  for (int c = 0; c < chunks; ++c) {
+    load(c);
+    hi = max(hi, n > 0 ? base + n - 1 : 0);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) hi = max(hi, __shfl_xor(hi, o, 64));
+  hi = __builtin_amdgcn_readfirstlane(hi);
+  while (lo < hi) {  // the largest key with more than i units at or above it
+    const int mid = (lo + hi + 1) >> 1;
+    if (count(mid) > i) lo = mid;
+    else hi = mid - 1;
+  }
+  int r = i - count(lo + 1);
+  for (int c = 0; c < chunks; ++c) {
+    load(c);
+    const bool has = lo >= base && lo < base + n;
+    const uint64_t m = __ballot(has);
+    const int here = __popcll(m);
+    if (r < here) {
+      const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+      const int l = __builtin_ctzll(__ballot(has && before == r));
+      u.seq = c * 64 + l;
+      u.unit = lo - __builtin_amdgcn_readlane(base, l);
+      u.row0 = __builtin_amdgcn_readlane(row0, l);
+      u.rows = __builtin_amdgcn_readlane(rows, l);
+      u.ctx = __builtin_amdgcn_readlane(ctx, l);
+      return u;
+    }
+    r -= here;
+  }
+  return u;
+}
+
 // ------------------------------------------------------------ fp32 MFMA tile kernel --
 //
 // The reference's element type.  fp32 MFMA (v_mfma_f32_32x32x2_f32) is 16x slower per flop
 // than bf16 and the kernel is bound by it.  Units are tiles of UR query rows of one sequence
 // for GW heads of one kv-head (as in prefill_mfma_kernel: GW = min(G, 4) heads, 4 / GW
-// subtiles of 32 rows); workgroup (group, s, r) of the grid takes the r-th, (r + R)-th, ... units
-// of sequence s from its end (R = gridDim.z).  Workgroups start in grid order as slots free up, so
-// the units with most keys start first and the short ones fill in behind them, and with the head
-// group as the fastest dimension a multiple of 8 groups keeps each kv-head's K/V on one die.  The
-// order before it, units ascending with the head group slowest, started the longest units last:
-// 5 prompts of 171 to 964 tokens at 32 / 8 heads of 64 took 177 us, 146
-// with the loop of that time.
+// subtiles of 32 rows); workgroup (group, i) of the grid takes the i-th unit of the batch, most keys
+// first (unit_by_work), and every gridDim.y-th after it.  Workgroups start in grid order as slots
+// free up, so the units with most keys start first and the short ones fill in behind them, and with
+// the head group as the fastest dimension a multiple of 8 groups keeps each kv-head's K/V on one
+// die.  Measured (kernel and cache write, us a call): 12 prompts of 128 to 2,048 tokens at head_dim
+// 128 1,749 with every sequence's units from its end, one sequence after the other, 1,370 sorted;
+// 16 prompts of 40 to 512 behind up to 1,000 cached at head_dim 64 390 -> 317; the 5 prompts below
+// 122.4 -> 114.6; one prompt of 40 rows the same (15.6).  The reversed second deal of unit_by_work
+// is the last 3 us of the 114.6, and 51.2 -> 46.2 for 3 prompts of 300 to 512.
 //
 //  * Bound: the fp32 MFMAs, 64 cycles each, 2 x D / 2 of them per tile.  The 32-key K and V tiles
 //    reach LDS by direct global -> LDS copies into two buffers each, K a tile further ahead than
@@ -1094,27 +1170,24 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int qi = lane & 31, h = lane >> 5;
-  const int s = blockIdx.y;
   const int G = a.num_heads / a.num_kv_heads;
   const int head = blockIdx.x * GW + (w % GW);
   const int kvh = (blockIdx.x * GW) / G;
   const int sub = w / GW;
-  const int row0 = a.cu_seqlens[s];
-  const int L = a.cu_seqlens[s + 1] - row0;
-  const int ctx = a.context_lens[s];
-  const int first = ctx - L;           // position of the sequence's first new row
   const float* q = static_cast<const float*>(a.q);
   const float* kc = static_cast<const float*>(a.k_cache);
   const float* vc = static_cast<const float*>(a.v_cache);
   float* out = static_cast<float*>(a.out);
-  const int32_t* bt = a.block_table + (int64_t)s * a.max_blocks;
   int bs = a.block_size;
   int key_cap = a.max_blocks * bs;  // positions the table row can address
-  int first_v = first;
-  // Per-lane arithmetic only: kept in VGPRs (the scalar registers are the tight budget here).
-  asm volatile("" : "+v"(bs), "+v"(key_cap), "+v"(first_v));
 
-  for (int unit = (L + UR - 1) / UR - 1 - (int)blockIdx.z; unit >= 0; unit -= gridDim.z) {
+  for (int i = blockIdx.y;; i += gridDim.y) {
+    const UnitAt at = unit_by_work(a.cu_seqlens, a.context_lens, a.num_seqs, UR, i, a.sched_cols);
+    if (at.seq < 0) break;
+    const int unit = at.unit, row0 = at.row0, L = at.rows, ctx = at.ctx;
+    const int first = ctx - L;           // position of the sequence's first new row
+    const int32_t* bt = a.block_table + (int64_t)at.seq * a.max_blocks;
+    int first_v = first;
     const int myrow = unit * UR + sub * kPT + qi;
     const bool row_ok = myrow < L;
     const int qpos = first_v + myrow;           // negative: a row without a position (zeros)
@@ -1214,11 +1287,12 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
     // Keys of tile kt that a row does not attend to, on the tiles that hold any.
     auto mask = [&](f32x16& st, int kt) __attribute__((always_inline)) {
       if (kt < kclear) return;
+      int key0 = kt * kPT + 4 * h;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int key = kt * kPT + 8 * j + 4 * h + r;
+          const int key = key0 + 8 * j + r;
           if (!row_ok || key > qpos || key >= nkeys) st[4 * j + r] = -INFINITY;
         }
     };
@@ -1487,8 +1561,10 @@ extern "C" int rg_prefill_packed(const void* query, const void* key_cache, const
       aligned16(value_cache) && aligned16(output) && stride % 4 == 0) {
     const int64_t UR = (int64_t)kPT * (kPWaves / GW);
     const int64_t qmax = std::min<int64_t>(std::max<int32_t>(max_query_len, 1), num_tokens);
-    const dim3 grid((unsigned)(num_heads / GW), (unsigned)num_seqs,
-                    (unsigned)std::min<int64_t>((qmax + UR - 1) / UR, 65535));
+    const int64_t groups = num_heads / GW, cus = device_cu_count();
+    if (cus % groups == 0 && head_dim <= 128) a.sched_cols = (int32_t)(cus / groups);  // (256: one workgroup per CU)
+    const int64_t items = (qmax + UR - 1) / UR * num_seqs, cols = std::max(a.sched_cols, 1);
+    const dim3 grid((unsigned)groups, (unsigned)std::min<int64_t>(ceil_div(items, cols) * cols, 65535));
     auto go = [&](auto dtag, auto gtag) {
       constexpr int D = decltype(dtag)::value;
       constexpr int W = decltype(gtag)::value;

@@ -237,6 +237,23 @@ def test_prefill_many_sequences(device, kernels, nseq):
     _run(device, kernels, w, seed=nseq + 1, check_seqs=list(range(0, nseq, 7)))
 
 
+@pytest.mark.parametrize("max_query_len", [None, 1])
+@pytest.mark.parametrize("nseq,H,Hkv,D", [(1, 32, 8, 64), (64, 8, 2, 64), (65, 8, 2, 64), (150, 6, 2, 128),
+                                          (9, 4, 4, 256)])
+def test_prefill_f32_units_by_work(device, kernels, nseq, H, Hkv, D, max_query_len):
+    """fp32 takes a batch's units from the one with most keys: one sequence, the edge of a 64-lane
+    chunk of sequences and past it, sequences without rows, more and fewer units than two per column
+    of workgroups, head counts with (8 groups) and without columns, an understated max_query_len."""
+    rng = np.random.default_rng(nseq)
+    lens = rng.integers(1, 100, nseq).astype(np.int32)
+    lens[1::5] = 0
+    prior = np.where(rng.random(nseq) < 0.5, rng.integers(1, 200, nseq), 0).astype(np.int32)
+    need = int(((prior + lens + 15) // 16).sum())
+    bt = wl.assign_blocks(prior + lens, 16, need + 8, 20, rng)
+    w = wl.PrefillWorkload(f"f32_{nseq}", "f32", H, Hkv, D, 16, need + 8, lens, bt, 5, prior=prior)
+    _run(device, kernels, w, seed=nseq + 1, max_query_len=max_query_len)
+
+
 def test_prefill_wide_table_rank_order(device, kernels):
     """A block table padded to 2200 entries (35,200 positions) puts the work-key bound past the
     sorted schedule's LDS table: the rank-order path, with prior context, bf16 D 128."""
