@@ -905,6 +905,7 @@ struct StreamArgs {
   int64_t kv_stride;
   int32_t table_stride;  // entries per block-table row (max_blocks counts 16-token sub-blocks)
   int32_t bs_shift;      // block_size = 16 << bs_shift
+  int32_t one_launch;    // 1: decode_short_kernel runs in place of the worker and merge kernels
   // Fused RoPE + cache write of the step's new tokens (decode_stream_kernel with ROPE): token s
   // is sequence s's; its k / v rows are [H_kv, D] at k_new / v_new + s H_kv D.
   const void* k_new;
@@ -1467,6 +1468,190 @@ __global__ __launch_bounds__(64 * G) void decode_stream_merge_kernel(StreamArgs 
   }
 }
 
+// ---------------------------------------------------------------- short -----
+//
+// Tables of few tokens (short_applies): one workgroup per segment (sequence, kv-head), kShortWaves
+// waves taking its 16-token sub-blocks in turn, their partials merged in LDS and the output written:
+// one launch and no scratch.  Such a call is bound by latency and launches, not by bytes: the
+// stream-K worker first finds its range by a scan over the context lengths, then its block-table
+// window, then its K/V rows, and the merge kernel follows.  Here the table entries (lane l of wave w
+// holds sub-block w + kShortWaves l), the context length and q are loaded at once, then the K/V
+// rows.  ROPE as in decode_stream_kernel: every wave rotates its q rows, the wave holding the last
+// sub-block writes and patches the new token's rows.
+// Measured (kernel trace, 4 sequences): 32 / 8 heads of 128 in bf16 at 100 tokens 7.8 us against 9.5 +
+// 3.4 of the two kernels and the gap between them, 11.3 against 8.9 + 3.8 at 400; fp32 heads of 64 at
+// 400 tokens 10.4 against 8.8 + 3.4.  Its slope is P.V on the VALU, ~1,100 cycles a sub-block and
+// wave; 16 tokens a wave more cost 1.1 us.
+constexpr int kShortWaves = 8;
+constexpr int kShortThreads = 64 * kShortWaves;
+constexpr int kShortMaxTokens = 16 * 64 * kShortWaves;  // one table entry per lane and wave
+
+template <typename T, int D, int G, bool ROPE>
+__global__ __launch_bounds__(kShortThreads) void decode_short_kernel(
+    StreamArgs a, const typename DecodeTileFor<T, D, G>::S* __restrict__ q_ptr,
+    const typename DecodeTileFor<T, D, G>::S* __restrict__ kc, const typename DecodeTileFor<T, D, G>::S* __restrict__ vc,
+    const int32_t* __restrict__ block_table, const int32_t* __restrict__ context_lens,
+    const int32_t* __restrict__ positions, const int32_t* __restrict__ slot_mapping) {
+  using Tile = DecodeTileFor<T, D, G>;
+  using S = typename Tile::S;
+  static_assert(!ROPE || !std::is_same_v<T, f32_t>, "the fused RoPE runs on the 16-bit tiles");
+  constexpr int GP = Tile::GP, HG = Tile::HG, NK = Tile::NK, NV = Tile::NV;
+  // Sub-blocks in flight ahead of the one computed (fp32 at head_dim 128: 64 registers each).
+  constexpr int AHEAD = std::is_same_v<T, f32_t> && D == 128 ? 1 : 2, NBUF = AHEAD + 1;
+  __shared__ float p_lds[kShortWaves][2][kBS * GP];
+  __shared__ float alpha_lds[kShortWaves][2][GP];
+  __shared__ float acc_lds[kShortWaves][G * D];
+  __shared__ float ml_lds[kShortWaves][2][GP];
+
+  const int kvh = blockIdx.x, s = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int H = a.num_heads, hkv = a.num_kv_heads;
+  const int sh = a.bs_shift, sub_mask = (1 << sh) - 1;
+
+  // Sub-block w + kShortWaves lane of the table row, within the row whatever the context is.
+  const int sb = w + kShortWaves * lane;
+  const int32_t* row = block_table + (int64_t)s * a.table_stride;
+  const int entry = sb < a.max_blocks ? row[sb >> sh] : 0;
+  const int ctx_raw = context_lens[s];
+  const S* qg = q_ptr + ((int64_t)s * H + (int64_t)kvh * G) * D;
+  Tile tile;
+  tile.init(lane);
+  tile.reset();
+
+  constexpr int QP = G * D <= 128 ? 1 : G * D <= 256 ? 2 : G * D <= 512 ? 4 : 8;
+  constexpr int KP = D / 2 >= 64 ? D / 128 : 1;
+  __shared__ __attribute__((aligned(16))) uint16_t rope_lds[ROPE ? kShortWaves : 1][ROPE ? G * D + D : 1];
+  uint16_t* const rq_lds = rope_lds[ROPE ? w : 0];
+  uint16_t* const rk_lds = rq_lds + G * D;
+  const int rq_p0 = lane * QP, rk_p0 = lane * KP;
+  RopeRun<T, QP> rq;
+  RopeRun<T, KP> rk;
+  uint4 vnew = make_uint4(0, 0, 0, 0);
+  int slot = -1;
+  if constexpr (ROPE) {
+    slot = slot_mapping[s];
+    const int pos = positions[s];  // (of a sequence without a context it is not used)
+    const float* cs = a.cos_sin + (int64_t)(ctx_raw > 0 ? pos : 0) * D;
+    if (rq_p0 < G * D / 2) rq.load(qg + (rq_p0 / (D / 2)) * D, cs, rq_p0 % (D / 2), D / 2);
+    const int64_t nrow = ((int64_t)s * hkv + kvh) * D;
+    if (rk_p0 < D / 2) rk.load(static_cast<const S*>(a.k_new) + nrow, cs, rk_p0, D / 2);
+    vnew = *reinterpret_cast<const uint4*>(static_cast<const S*>(a.v_new) + nrow + tile.vd0);
+  } else {
+    tile.load_q(qg);
+  }
+
+  const int ctx = max(0, min(ctx_raw, a.max_blocks * kBS));
+  const int nblk = (ctx + kBS - 1) / kBS;
+  const int nb = w < nblk ? (nblk - w + kShortWaves - 1) / kShortWaves : 0;  // this wave's sub-blocks
+  if (nb > 0) {
+    const int64_t head = (int64_t)kvh * (kBS << sh) * D;
+    uint4 kbuf[NBUF][NK], vbuf[NBUF][NV];
+    auto load_block = [&](int j, uint4 (&kk)[NK], uint4 (&vv)[NV]) __attribute__((always_inline)) {
+      const int e = __builtin_amdgcn_readlane(entry, j);
+      const int64_t off = (int64_t)e * a.kv_stride + head + (int64_t)((w + kShortWaves * j) & sub_mask) * (kBS * D);
+      tile.template load_part<1, 0>(kc + off, vc + off, kk, vv);
+    };
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) load_block(min(u, nb - 1), kbuf[u], vbuf[u]);
+    int patch_j = -1;  // the sub-block of this wave that takes the new token's rows
+    if constexpr (ROPE) {
+      if (rq_p0 < G * D / 2) rq.rotate_to(rq_lds + (rq_p0 / (D / 2)) * D, rq_p0 % (D / 2), D / 2);
+      const int p = ctx_raw - 1, pb = p >> 4;  // the new token's position and sub-block
+      if (slot >= 0 && p >= 0 && p < a.max_blocks * kBS && pb % kShortWaves == w) {
+        const int e = __builtin_amdgcn_readlane(entry, pb / kShortWaves);
+        if (((e << sh) | (pb & sub_mask)) * kBS + (p & (kBS - 1)) == slot) {
+          patch_j = pb / kShortWaves;
+          if (rk_p0 < D / 2) rk.rotate_to(rk_lds, rk_p0, D / 2);
+        }
+      }
+      wave_lds_sync();
+      const uint4* qrow = reinterpret_cast<const uint4*>(rq_lds + (tile.col % G) * D + 8 * tile.seg);
+#pragma unroll
+      for (int i = 0; i < NK; ++i) tile.qa[i] = qrow[4 * i];
+    }
+    // Every step issues a sub-block's loads (the last one again past the end), so that the
+    // compiler's waits are exact counts.
+    for (int j0 = 0; j0 < nb; j0 += NBUF) {
+#pragma unroll
+      for (int u = 0; u < NBUF; ++u) {
+        const int j = j0 + u;
+        if (j < nb) {
+          load_block(min(j + AHEAD, nb - 1), kbuf[(u + AHEAD) % NBUF], vbuf[(u + AHEAD) % NBUF]);
+          if constexpr (ROPE) {
+            if (j == patch_j) {
+              uint4 knew[NK];
+              const uint4* krow = reinterpret_cast<const uint4*>(rk_lds + 8 * tile.seg);
+#pragma unroll
+              for (int i = 0; i < NK; ++i) knew[i] = krow[4 * i];
+              tile.template patch<1>(kbuf[u], vbuf[u], 0, slot & (kBS - 1), knew, vnew);
+              const int bsz = kBS << sh;
+              const int64_t nrow = (int64_t)(slot >> (4 + sh)) * a.kv_stride +
+                                   ((int64_t)kvh * bsz + (slot & (bsz - 1))) * D;
+              S* kdst = const_cast<S*>(kc) + nrow;
+              S* vdst = const_cast<S*>(vc) + nrow;
+              if (tile.col == 0) {
+#pragma unroll
+                for (int i = 0; i < NK; ++i) *reinterpret_cast<uint4*>(kdst + 32 * i + 8 * tile.seg) = knew[i];
+              }
+              if (tile.vrow == 0) *reinterpret_cast<uint4*>(vdst + tile.vd0) = vnew;
+            }
+          }
+          tile.step(kbuf[u], vbuf[u], (w + kShortWaves * j) * kBS, ctx, a.scale_log2, p_lds[w][j & 1],
+                    alpha_lds[w][j & 1]);
+        }
+      }
+    }
+  }
+
+  float lsum[4];
+  tile.reduce(lsum);
+  if (tile.vrow == 0) {
+#pragma unroll
+    for (int h = 0; h < G; ++h) {
+      float4* dst = reinterpret_cast<float4*>(&acc_lds[w][h * D + tile.vd0]);
+#pragma unroll
+      for (int q4 = 0; q4 < Tile::ACC / 4; ++q4)
+        dst[q4] = make_float4(tile.acc[h][4 * q4], tile.acc[h][4 * q4 + 1], tile.acc[h][4 * q4 + 2],
+                              tile.acc[h][4 * q4 + 3]);
+    }
+  }
+  if (tile.seg < HG && tile.col == 0) {
+    *reinterpret_cast<float4*>(&ml_lds[w][0][4 * tile.seg]) =
+        make_float4(tile.m_run[0], tile.m_run[1], tile.m_run[2], tile.m_run[3]);
+    *reinterpret_cast<float4*>(&ml_lds[w][1][4 * tile.seg]) = make_float4(lsum[0], lsum[1], lsum[2], lsum[3]);
+  }
+  __syncthreads();
+
+  // Merge the waves and write out two consecutive dims per thread (zeros without a context).
+  for (int idx = threadIdx.x; idx < G * D / 2; idx += kShortThreads) {
+    const int h = idx / (D / 2);
+    const int d = (idx % (D / 2)) * 2;
+    float M = -INFINITY;
+#pragma unroll
+    for (int ww = 0; ww < kShortWaves; ++ww) M = fmaxf(M, ml_lds[ww][0][h]);
+    float L = 0.f, o0 = 0.f, o1 = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < kShortWaves; ++ww) {
+      const float mw = ml_lds[ww][0][h];
+      const float f = mw == -INFINITY ? 0.f : exp2f(mw - M);
+      const float2 o = *reinterpret_cast<const float2*>(&acc_lds[ww][h * D + d]);
+      L += f * ml_lds[ww][1][h];
+      o0 += f * o.x;
+      o1 += f * o.y;
+    }
+    const float inv = L != 0.f ? 1.f / L : 1.f;
+    auto* op = static_cast<typename elem<T>::storage*>(a.out) + ((int64_t)s * H + (int64_t)kvh * G + h) * D + d;
+    if constexpr (std::is_same_v<T, f32_t>) {
+      op[0] = o0 * inv;
+      op[1] = o1 * inv;
+    } else {
+      *reinterpret_cast<uint32_t*>(op) =
+          (uint32_t)elem<T>::from_f32(o0 * inv) | ((uint32_t)elem<T>::from_f32(o1 * inv) << 16);
+    }
+  }
+}
+
 // ---------------------------------------------------------------- merge -----
 
 struct MergeArgs {
@@ -1801,9 +1986,37 @@ size_t stream_bytes(const Shape& sh, int32_t workers, StreamScratch* carve, void
   return acc + ml + desc;
 }
 
+// Whether the one-launch kernel takes the call: G 1 to 8 at head_dim 64 or 128, at most 256 KB of K
+// and V in a segment's table row (one CU streams a segment at ~41 GB/s here; at 400 KB the two
+// kernels together are as fast on the device, and at 800 KB 5 us faster) and at most 64 MB in the
+// whole table (64 sequences of 400 tokens at 8 kv-heads of 128, 105 MB: 32.6 us a pass of RoPE and
+// decode against 26.5; 16 of 800, 52 MB: 23.8 against 26.1).  The table's width stands for the
+// contexts, which the host does not know: contexts shorter than it only make the call shorter.
+#ifndef RG_SHORT_KB
+#define RG_SHORT_KB 256
+#endif
+#ifndef RG_SHORT_TOTAL_MB
+#define RG_SHORT_TOTAL_MB 64
+#endif
+bool short_applies(const Shape& sh, int elem_bytes) {
+  const int64_t tokens = (int64_t)sh.MB * sh.bs, segment = tokens * sh.D * 2 * elem_bytes;
+  return (sh.D == 64 || sh.D == 128) && sh.H / sh.Hkv <= 8 && tokens <= kShortMaxTokens &&
+         segment <= (int64_t)RG_SHORT_KB << 10 && segment * sh.B * sh.Hkv <= (int64_t)RG_SHORT_TOTAL_MB << 20 &&
+         sh.B <= 65535;
+}
+
 template <typename T, int D, int G, bool ROPE = false>
 void launch_stream(const StreamArgs& sa, const DecodeArgs& a, hipStream_t s) {
   using S = typename DecodeTileFor<T, D, G>::S;
+  if constexpr (D <= 128 && G <= 8) {
+    if (sa.one_launch) {
+      hipLaunchKernelGGL((decode_short_kernel<T, D, G, ROPE>), dim3(sa.num_kv_heads, sa.batch), dim3(kShortThreads), 0,
+                         s, sa, static_cast<const S*>(a.q), static_cast<const S*>(a.k_cache),
+                         static_cast<const S*>(a.v_cache), a.block_table, a.context_lens, sa.positions,
+                         sa.slot_mapping);
+      return;
+    }
+  }
   hipLaunchKernelGGL((decode_stream_kernel<T, D, G, ROPE>), dim3(sa.num_workers), dim3(64), 0, s, sa,
                      static_cast<const S*>(a.q), static_cast<const S*>(a.k_cache),
                      static_cast<const S*>(a.v_cache), a.block_table, a.context_lens, sa.positions,
@@ -1886,6 +2099,7 @@ int run_stream(const char* op, const DecodeArgs& a, int32_t dtype, const Shape& 
   sa.kv_stride = a.kv_stride;
   sa.table_stride = sh.MB;
   sa.bs_shift = a.bs_shift;
+  sa.one_launch = short_applies(sh, dtype_bytes(dtype)) ? 1 : 0;
   const int G = sh.H / sh.Hkv;
   if (rope != nullptr) {
     sa.k_new = rope->k;

@@ -603,3 +603,29 @@ def test_stream_random_shapes(device, kernels):
         got = gpu_v1(kernels, inp, True)
         assert not np.isnan(got).any(), f"case {case}"
         assert_close(got, want, dt, f"case {case}: B={B} G={G} Hkv={Hkv} D={D} bs={bs} {dt}")
+
+
+SHORT_EDGES = [0, 1, 15, 16, 17, 127, 128, 129, 255, 256, 257]  # sub-block and wave-turn edges
+
+
+@pytest.mark.parametrize("dt,D,bs,mb", [
+    ("bf16", 128, 16, 32), ("bf16", 128, 16, 33),   # 256 KB of K/V per segment: the one-launch kernel; past it
+    ("f16", 64, 32, 32), ("f16", 64, 32, 33), ("f32", 64, 16, 32), ("f32", 128, 16, 16), ("f32", 128, 64, 4)])
+@pytest.mark.parametrize("G", [1, 3, 4, 8])
+def test_decode_short_tables(device, kernels, dt, D, bs, mb, G):
+    """Tables of few tokens (decode_short_kernel) at the edges of its waves' turns, up to the whole
+    table, without a context, and one block past the widest table it takes; fused pool."""
+    cap = mb * bs
+    ctx = [c for c in SHORT_EDGES if c <= cap] + [cap - 1, cap]
+    inp = make_inputs(device, ctx, dt, H=2 * G, Hkv=2, D=D, bs=bs, seed=mb + G, fused=True, mb=mb)
+    got = gpu_v1(kernels, inp, workspace=True)
+    assert_close(got, oracle_v1_plus(inp), dt, f"{dt} D {D} bs {bs} mb {mb} G {G}")
+    np.testing.assert_array_equal(got[0], 0)
+
+
+@pytest.mark.parametrize("batch", [64, 65])
+def test_decode_short_tables_total(device, kernels, batch):
+    """At and past 64 MB of K/V in the whole table (8 kv-heads of 64 in fp32, 256 tokens each)."""
+    rng = np.random.default_rng(batch)
+    inp = make_inputs(device, rng.integers(0, 257, batch), "f32", H=16, Hkv=8, D=64, seed=batch, mb=16)
+    assert_close(gpu_v1(kernels, inp, workspace=True), oracle_v1_plus(inp), "f32", f"batch {batch}")
