@@ -42,7 +42,9 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream of t's device as a hipStream_t (without building a torch.cuda.Stream:
+    2 us of the host's time per launch, which small calls are bound by)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _require_cuda(*tensors: Optional[torch.Tensor]) -> None:
@@ -72,12 +74,13 @@ def cache_geometry(k_cache: torch.Tensor, v_cache: torch.Tensor) -> tuple[int, i
                            f"caches must be [num_blocks, num_kv_heads, block_size, head_dim], got "
                            f"{tuple(k_cache.shape)} and {tuple(v_cache.shape)}")
     _, hkv, bs, d = k_cache.shape
-    for c in (k_cache, v_cache):
-        if c.stride(3) != 1 or c.stride(2) != d or c.stride(1) != bs * d:
-            raise RailgunError(_lib.RG_ERR_INVALID_ARGUMENT, "cache blocks must be contiguous [H_kv, bs, D]")
-    if k_cache.stride(0) != v_cache.stride(0) or k_cache.dtype != v_cache.dtype:
+    k_stride, v_stride = k_cache.stride(), v_cache.stride()
+    inner = (bs * d, d, 1)
+    if k_stride[1:] != inner or v_stride[1:] != inner:
+        raise RailgunError(_lib.RG_ERR_INVALID_ARGUMENT, "cache blocks must be contiguous [H_kv, bs, D]")
+    if k_stride[0] != v_stride[0] or k_cache.dtype != v_cache.dtype:
         raise RailgunError(_lib.RG_ERR_INVALID_ARGUMENT, "k and v caches must share dtype and block stride")
-    return int(hkv), int(bs), int(d), int(k_cache.stride(0))
+    return hkv, bs, d, k_stride[0]
 
 
 def rope_cos_sin_table(max_position: int, head_dim: int, theta: float,
@@ -405,7 +408,7 @@ class PagedAttentionOp:
             raise RailgunError(_lib.RG_ERR_INVALID_ARGUMENT,
                                f"cache has {num_kv_heads} kv heads, op expects {self.num_kv_heads}")
         max_blocks = int(block_table.shape[1])
-        out = torch.zeros_like(q)
+        out = torch.empty_like(q)  # every route writes every row, zeros for an empty context
         k = self.kernels
         if max_context_len <= V1_MAX_CONTEXT:
             ws_bytes = k.v1_workspace_bytes(batch, num_heads, self.num_kv_heads, head_dim, block_size, max_blocks)

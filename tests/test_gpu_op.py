@@ -127,3 +127,30 @@ def test_argument_errors(device, kernels):
         kernels.launch_v1(q2, kc2, kc2, bt2, cl, q2, 1.0, 4, 3, 64, 16, 64, 1)
     with pytest.raises(RailgunError, match="workspace"):
         kernels.launch_v1(q2, kc2, kc2, bt2, cl, q2, 1.0, 4, 4, 64, 16, 64, 1, workspace=ws)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("H,Hkv,D,bs,mb", [(8, 2, 64, 16, 8), (8, 2, 64, 16, 200), (8, 2, 64, 16, 400),
+                                           (16, 1, 256, 16, 8), (4, 2, 80, 16, 8), (4, 2, 80, 16, 400),
+                                           (4, 2, 64, 8, 20), (4, 2, 64, 8, 700)])
+def test_execute_writes_every_row(device, kernels, dt, H, Hkv, D, bs, mb):
+    """execute's output is not cleared beforehand: rows of sequences without a context come out as
+    zeros on every route (one launch, stream-K, v2, the generic kernels), also out of memory that
+    held NaN, and the others as attention."""
+    rng = np.random.default_rng(mb + D)
+    ctx = np.array([0, 33, 0, mb * bs, 1], np.int32)
+    nb = mb + 8
+    bt = rng.permutation(nb)[:mb].astype(np.int32)[None].repeat(len(ctx), 0)
+    q = normal(rng, (len(ctx), H, D), dt)
+    kc, vc = normal(rng, (nb, Hkv, bs, D), dt), normal(rng, (nb, Hkv, bs, D), dt)
+    op = PagedAttentionOp(D ** -0.5, H, Hkv, D, bs, kernels)
+    dq = to_dev(q, dt, device)
+    args = (dq, to_dev(kc, dt, device), to_dev(vc, dt, device), i32(bt, device), i32(ctx, device))
+    for _ in range(3):
+        held = [torch.full_like(dq, float("nan")) for _ in range(4)]
+        del held
+        out = op.execute(*args, None, int(ctx.max()))
+        torch.cuda.synchronize()
+        got = dev_f32(out)
+        np.testing.assert_array_equal(got[[0, 2]], 0)
+        assert_close(got, orc.paged_attention_v1_plus(q, kc, vc, bt, ctx, op.scale, dt), dt)
