@@ -146,6 +146,25 @@ def test_linear_split_k(device, M, N, K):
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 14336), (27, 4096, 14336), (64, 4096, 14336), (16, 3072, 8192),
+                                   (27, 4096, 4096), (5, 3072, 3072)])
+def test_linear_splits_long_walks(device, M, N, K, dt):
+    """Layers whose workgroups would walk many chunks in turn split K too (rows of one and of several
+    row tiles): linear and linear_residual against fp32, repeated calls bit-identical."""
+    ws_bytes = linear_workspace_bytes(M, N, K)
+    assert ws_bytes > 0, "split on a 256-CU device"
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=device).to(TORCH[dt])
+    w = (0.02 * torch.randn(N, K, generator=g, device=device)).to(TORCH[dt])
+    r = torch.randn(M, N, generator=g, device=device).to(TORCH[dt])
+    ws = torch.full((ws_bytes,), 0xFF, dtype=torch.uint8, device=device)   # NaN-filled: every partial is written
+    out, again, res = linear(x, w, workspace=ws), linear(x, w, workspace=ws), linear_residual(x, w, r.clone(), ws)
+    _check(out, x, w, f"{M}x{N}x{K} {dt}", ref_on_device=True)
+    assert torch.equal(again.view(torch.int16), out.view(torch.int16)), "split K not deterministic"
+    assert torch.equal(res, (r.float() + out.float()).to(TORCH[dt])), "the residual add of the rounded sum"
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("M,I,K", [(128, 8192, 2048), (1, 8192, 2048), (37, 512, 256), (100, 1040, 1024)])
 def test_linear_silu_mul(device, M, I, K, dt):
     """The gate/up projection with SiLU·mul in the epilogue against the fp32 products rounded the
