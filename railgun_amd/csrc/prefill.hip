@@ -272,6 +272,81 @@ template <> __device__ __forceinline__ float pair_sum<f16_t>(uint32_t pair, floa
                                 acc, false);
 }
 
+// The i-th of a batch's units of UR rows, most keys first: unit u of a sequence whose first new row
+// sits at position `first` has the work key floor(max(first, 0) / UR) + u, so a key occurs at most
+// once per sequence, and the units of at least a given key are counted with one sum over the
+// sequences (one per lane, 64 at a time): a binary search over the keys, then the sequences of the
+// key found in order.  Returned wave-uniform; seq = -1 past the last
+// unit; total is their number.
+// With cols > 0 the first 2 cols units start at once and workgroups i and i + cols share a CU: the
+// second cols units are dealt in reverse, so that the longest of them go with the shortest of the
+// first.
+struct UnitAt { int seq, unit, row0, rows, ctx, total; };
+__device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t* ctx_lens, int num_seqs, int UR,
+                                               int i, int cols) {
+  const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+  int c_loaded = -1, row0 = 0, rows = 0, ctx = 0, base = 0, n = 0;
+  auto load = [&](int c) {  // the sequences of chunk c, one per lane
+    if (c == c_loaded) return;
+    c_loaded = c;
+    const int s = c * 64 + lane;
+    row0 = rows = ctx = base = n = 0;
+    if (s < num_seqs) {
+      row0 = cu[s];
+      rows = cu[s + 1] - row0;
+      ctx = ctx_lens[s];
+      n = rows > 0 ? (rows + UR - 1) / UR : 0;
+      base = max(ctx - rows, 0) / UR;
+    }
+  };
+  const int chunks = (num_seqs + 63) / 64;
+  auto sum = [](int v) { return __builtin_amdgcn_readlane(wave_prefix_sum(v), 63); };
+  auto count = [&](int k) {  // units whose key is at least k
+    int t = 0;
+    for (int c = 0; c < chunks; ++c) {
+      load(c);
+      t += sum(min(max(base + n - k, 0), n));
+    }
+    return t;
+  };
+  UnitAt u{-1, 0, 0, 0, 0, 0};
+  const int total = u.total = count(0);
+  if (i >= cols && i < 2 * cols) i = 3 * cols - 1 - i;
+  if (i >= total) return u;
+  int lo = 0, hi = 0;
+  for (int c = 0; c < chunks; ++c) {
+    load(c);
+    hi = max(hi, n > 0 ? base + n - 1 : 0);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) hi = max(hi, __shfl_xor(hi, o, 64));
+  hi = __builtin_amdgcn_readfirstlane(hi);
+  while (lo < hi) {  // the largest key with more than i units at or above it
+    const int mid = (lo + hi + 1) >> 1;
+    if (count(mid) > i) lo = mid;
+    else hi = mid - 1;
+  }
+  int r = i - count(lo + 1);
+  for (int c = 0; c < chunks; ++c) {
+    load(c);
+    const bool has = lo >= base && lo < base + n;
+    const uint64_t m = __ballot(has);
+    const int here = __popcll(m);
+    if (r < here) {
+      const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+      const int l = __builtin_ctzll(__ballot(has && before == r));
+      u.seq = c * 64 + l;
+      u.unit = lo - __builtin_amdgcn_readlane(base, l);
+      u.row0 = __builtin_amdgcn_readlane(row0, l);
+      u.rows = __builtin_amdgcn_readlane(rows, l);
+      u.ctx = __builtin_amdgcn_readlane(ctx, l);
+      return u;
+    }
+    r -= here;
+  }
+  return u;
+}
+
 // LDS image of one key tile (two KV blocks of 16 keys).  K: the 16-byte chunk c of key k of
 // block b at b * KBYTES / 2 + c * 256 + k * 16, so that one copy instruction (1 KB: chunks
 // 4n .. 4n+3 of the block's 16 keys) reads from one block only, and the MFMA A-operand read
@@ -292,8 +367,10 @@ struct PTile {
   __device__ static __forceinline__ int vchunk(int key, int c) { return c ^ (2 * (key & 3)); }
 };
 
-template <typename T, int D, int GW>
-__global__ __launch_bounds__(kPThreads, pf_wg_per_cu<D>()) void prefill_mfma_kernel(
+// DIRECT: few units, at most one per workgroup of a head group (more only when max_query_len
+// understates a sequence): workgroup q takes the q-th by work (unit_by_work) and builds no tables.
+template <typename T, int D, int GW, bool DIRECT = false>
+__global__ __launch_bounds__(kPThreads, DIRECT ? 2 : pf_wg_per_cu<D>()) void prefill_mfma_kernel(
     PrefillArgs a, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc,
     const uint16_t* __restrict__ vc, const int32_t* __restrict__ block_table,
     const int32_t* __restrict__ context_lens, const int32_t* __restrict__ cu_seqlens) {
@@ -343,7 +420,7 @@ __global__ __launch_bounds__(kPThreads, pf_wg_per_cu<D>()) void prefill_mfma_ker
   const int kvh = grp % hkv;
   const int nq_wg = gridDim.x / ngroups;
   const int qw = blockIdx.x / ngroups;
-  const bool sorted = a.sched_kbound > 0;
+  const bool sorted = !DIRECT && a.sched_kbound > 0;
   const int kb = a.sched_kbound;  // sorted schedule: keys live in [1, kb]
   const int table_tokens = a.max_blocks * a.block_size;
   const int H = a.num_heads;
@@ -450,6 +527,7 @@ __global__ __launch_bounds__(kPThreads, pf_wg_per_cu<D>()) void prefill_mfma_ker
   struct Unit {
     int s, t, t_stop, row0, L, prior;
   };
+  __shared__ int2 sched_next[kPWaves];  // DIRECT
   // Item u -> its first unit; false for an item without a tile (rank order).
   auto resolve = [&](int u, Unit& un) -> bool {
     if (sorted) {
@@ -486,6 +564,19 @@ __global__ __launch_bounds__(kPThreads, pf_wg_per_cu<D>()) void prefill_mfma_ker
       un.L = __builtin_amdgcn_readfirstlane(sched_seq[un.s + 1].x) - un.row0;
       un.prior = __builtin_amdgcn_readfirstlane(m0.y);
       un.t = k - seq_keys(un.L, un.prior).x;
+      un.t_stop = un.t - 1;
+      return true;
+    }
+    if constexpr (DIRECT) {
+      const UnitAt at = unit_by_work(cu_seqlens, context_lens, a.num_seqs, UR, u, 0);
+      // The next item and their number wait in LDS, not in scalar registers (at their limit).
+      sched_next[w] = make_int2(u + (int)(gridDim.x / ngroups), at.total);
+      if (at.seq < 0) return false;
+      un.s = at.seq;
+      un.row0 = at.row0;
+      un.L = at.rows;
+      un.prior = min(at.ctx, table_tokens) - at.rows;
+      un.t = at.unit;
       un.t_stop = un.t - 1;
       return true;
     }
@@ -588,7 +679,9 @@ __global__ __launch_bounds__(kPThreads, pf_wg_per_cu<D>()) void prefill_mfma_ker
 
   Unit cur{};
   bool have = false;
-  if (cols > 0) {
+  if constexpr (DIRECT) {
+    have = resolve(qw, cur);
+  } else if (cols > 0) {
     const int col = qw % cols, slot = qw / cols;
     const int u = slot * cols + ((slot & 1) ? cols - 1 - col : col);  // round `slot` of the column
     have = u < n_items && resolve(u, cur);
@@ -927,7 +1020,7 @@ __global__ __launch_bounds__(kPThreads, pf_wg_per_cu<D>()) void prefill_mfma_ker
     nxt = cur;
     nxt.t = cur.t - 1;
     nhave = true;
-  } else {
+  } else if constexpr (!DIRECT) {
     for (int u = take_item(); u < n_items; u = take_item()) {
       if (resolve(u, nxt)) {
         nhave = true;
@@ -1034,83 +1127,16 @@ __global__ __launch_bounds__(kPThreads, pf_wg_per_cu<D>()) void prefill_mfma_ker
       wave_lds_fence();  // the reads have returned before the next pass overwrites the buffer
     }
   }
-  cur = nxt;
-  have = nhave;
+  if constexpr (DIRECT) {  // (found here, past the unit's live state: a second unit is the exception)
+    const int2 nx = sched_next[w];
+    have = __builtin_amdgcn_readfirstlane(nx.x) < __builtin_amdgcn_readfirstlane(nx.y) &&
+           resolve(__builtin_amdgcn_readfirstlane(nx.x), cur);
+    if (have) load_unit(cur);
+  } else {
+    cur = nxt;
+    have = nhave;
+  }
   }  // units of this workgroup
-}
-
-// The i-th of a batch's units of UR rows, most keys first: unit u of a sequence whose first new row
-// sits at position `first` has the work key floor(max(first, 0) / UR) + u, so a key occurs at most
-// once per sequence, and the units of at least a given key are counted with one sum over the
-// sequences (one per lane, 64 at a time): a binary search over the keys, then the sequences of the
-// key found in order.  Returned wave-uniform; seq = -1 past the last unit.
-// With cols > 0 the first 2 cols units start at once and workgroups i and i + cols share a CU: the
-// second cols units are dealt in reverse, so that the longest of them go with the shortest of the
-// first.
-struct UnitAt { int seq, unit, row0, rows, ctx; };
-__device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t* ctx_lens, int num_seqs, int UR,
-                                               int i, int cols) {
-  const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
-  int c_loaded = -1, row0 = 0, rows = 0, ctx = 0, base = 0, n = 0;
-  auto load = [&](int c) {  // the sequences of chunk c, one per lane
-    if (c == c_loaded) return;
-    c_loaded = c;
-    const int s = c * 64 + lane;
-    row0 = rows = ctx = base = n = 0;
-    if (s < num_seqs) {
-      row0 = cu[s];
-      rows = cu[s + 1] - row0;
-      ctx = ctx_lens[s];
-      n = rows > 0 ? (rows + UR - 1) / UR : 0;
-      base = max(ctx - rows, 0) / UR;
-    }
-  };
-  const int chunks = (num_seqs + 63) / 64;
-  auto sum = [](int v) { return __builtin_amdgcn_readlane(wave_prefix_sum(v), 63); };
-  auto count = [&](int k) {  // units whose key is at least k
-    int t = 0;
-    for (int c = 0; c < chunks; ++c) {
-      load(c);
-      t += sum(min(max(base + n - k, 0), n));
-    }
-    return t;
-  };
-  UnitAt u{-1, 0, 0, 0, 0};
-  const int total = count(0);
-  if (i >= cols && i < 2 * cols) i = 3 * cols - 1 - i;
-  if (i >= total) return u;
-  int lo = 0, hi = 0;
-  for (int c = 0; c < chunks; ++c) {
-    load(c);
-    hi = max(hi, n > 0 ? base + n - 1 : 0);
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) hi = max(hi, __shfl_xor(hi, o, 64));
-  hi = __builtin_amdgcn_readfirstlane(hi);
-  while (lo < hi) {  // the largest key with more than i units at or above it
-    const int mid = (lo + hi + 1) >> 1;
-    if (count(mid) > i) lo = mid;
-    else hi = mid - 1;
-  }
-  int r = i - count(lo + 1);
-  for (int c = 0; c < chunks; ++c) {
-    load(c);
-    const bool has = lo >= base && lo < base + n;
-    const uint64_t m = __ballot(has);
-    const int here = __popcll(m);
-    if (r < here) {
-      const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-      const int l = __builtin_ctzll(__ballot(has && before == r));
-      u.seq = c * 64 + l;
-      u.unit = lo - __builtin_amdgcn_readlane(base, l);
-      u.row0 = __builtin_amdgcn_readlane(row0, l);
-      u.rows = __builtin_amdgcn_readlane(rows, l);
-      u.ctx = __builtin_amdgcn_readlane(ctx, l);
-      return u;
-    }
-    r -= here;
-  }
-  return u;
 }
 
 // ------------------------------------------------------------ fp32 MFMA tile kernel --
@@ -1520,10 +1546,17 @@ extern "C" int rg_prefill_packed(const void* query, const void* key_cache, const
     const int64_t per_group =
         std::min<int64_t>(items, std::max<int64_t>(1, wg_per_cu * device_cu_count() / ngroups));
     const dim3 grid((unsigned)(per_group * ngroups));
+    // Few units, at most two per CU: the form without schedule tables, whose set-up takes ~1 us less
+    // of a call bound by it (RoPE + cache and prefill, us: 9 fp16 prompts of 33 to 149 tokens at 24 /
+    // 8 heads of 128 14.2 -> 13.35, 16 of up to 64 at 28 / 4 15.0 -> 14.05, one of 500 at 32 / 8 heads
+    // of 64 14.4 -> 14.05).  Not at head_dim 128 with four heads per workgroup over long tables: its
+    // tile loop there is 1.3 % slower (one prompt of 2,000 tokens 41.0 against 41.6).
+    const bool direct = items <= 2 * device_cu_count() / ngroups && head_dim <= 128 &&
+                        (head_dim == 64 || GW < 4 || (int64_t)max_blocks_per_seq * block_size <= 512);
     // Columns: every CU holds three workgroups of one head group (workgroup b shares its CU with
     // b +- cu_count, measured), i.e. the group's workgroups q, q + C, q + 2C with C = cu / groups.
     const int64_t cus = device_cu_count();
-    if (RG_PF_WEIGHTED && wg_per_cu == 3 && a.sched_kbound > 0 && cus % ngroups == 0 &&
+    if (RG_PF_WEIGHTED && !direct && wg_per_cu == 3 && a.sched_kbound > 0 && cus % ngroups == 0 &&
         per_group == 3 * (cus / ngroups)) {
       a.sched_cols = (int32_t)(cus / ngroups);
     }
@@ -1531,9 +1564,15 @@ extern "C" int rg_prefill_packed(const void* query, const void* key_cache, const
       using T = decltype(tag);
       constexpr int D = decltype(dtag)::value;
       constexpr int W = decltype(gtag)::value;
-      hipLaunchKernelGGL((prefill_mfma_kernel<T, D, W>), grid, dim3(kPThreads), 0, s, a,
-                         static_cast<const uint16_t*>(query), static_cast<const uint16_t*>(key_cache),
-                         static_cast<const uint16_t*>(value_cache), block_table, context_lens, cu_seqlens);
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kPThreads), 0, s, a, static_cast<const uint16_t*>(query),
+                           static_cast<const uint16_t*>(key_cache), static_cast<const uint16_t*>(value_cache),
+                           block_table, context_lens, cu_seqlens);
+      };
+      if constexpr (D <= 128) {
+        if (direct) return launch(prefill_mfma_kernel<T, D, W, true>);
+      }
+      launch(prefill_mfma_kernel<T, D, W>);
     };
     auto go_gw = [&](auto tag, auto dtag) {
       if (GW == 4) go(tag, dtag, std::integral_constant<int, 4>{});

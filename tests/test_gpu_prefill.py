@@ -254,6 +254,19 @@ def test_prefill_f32_units_by_work(device, kernels, nseq, H, Hkv, D, max_query_l
     _run(device, kernels, w, seed=nseq + 1, max_query_len=max_query_len)
 
 
+@pytest.mark.parametrize("max_query_len", [None, 1])
+@pytest.mark.parametrize("dt,G,D,lens,prior", [
+    ("bf16", 4, 128, [33, 1, 0, 150, 97], [0, 40, 7, 0, 300]),     # tables up to 512 tokens
+    ("f16", 3, 128, [33, 1, 0, 150, 97], [0, 40, 7, 0, 1300]),
+    ("bf16", 1, 64, [256, 5], [0, 900]), ("f16", 8, 64, [1], [0]), ("bf16", 2, 128, [129, 128, 127], [0, 0, 64]),
+    ("bf16", 4, 64, [7] * 15 + [0], [11] * 16)])
+def test_prefill_few_units(device, kernels, dt, G, D, lens, prior, max_query_len):
+    """At most two units per CU: the form without schedule tables, with sequences without rows, and
+    with an understated max_query_len (one workgroup per head group then walks every unit)."""
+    w = _gqa_workload(G, D, lens, prior, seed=len(lens) + D, dt=dt, H=8 * G)
+    _run(device, kernels, w, seed=G + D, max_query_len=max_query_len)
+
+
 def test_prefill_wide_table_rank_order(device, kernels):
     """A block table padded to 2200 entries (35,200 positions) puts the work-key bound past the
     sorted schedule's LDS table: the rank-order path, with prior context, bf16 D 128."""
