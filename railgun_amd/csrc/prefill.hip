@@ -275,49 +275,60 @@ template <> __device__ __forceinline__ float pair_sum<f16_t>(uint32_t pair, floa
 // The i-th of a batch's units of UR rows, most keys first: unit u of a sequence whose first new row
 // sits at position `first` has the work key floor(max(first, 0) / UR) + u, so a key occurs at most
 // once per sequence, and the units of at least a given key are counted with one sum over the
-// sequences (one per lane, 64 at a time): a binary search over the keys, then the sequences of the
-// key found in order.  Returned wave-uniform; seq = -1 past the last
-// unit; total is their number.
+// sequences, kUnitChunks to a lane and all loaded at once: a binary search over the keys, then the
+// sequences of the key found in order.  Returned wave-uniform; seq = -1 past the last unit; total
+// is their number.
 // With cols > 0 the first 2 cols units start at once and workgroups i and i + cols share a CU: the
 // second cols units are dealt in reverse, so that the longest of them go with the shortest of the
 // first.
+// More than kUnitSeqs sequences would have to be read again at every step of the search, a round
+// trip each (fp32 prompts of up to 40 rows, 32 / 8 heads of 64, 64 sequences to a read: 256 of them
+// 76.5 us against 61.0 so, 1,000 562.7): no search then, item i is the (i / num_seqs)-th unit from
+// the end of sequence i % num_seqs, and the caller steps by a multiple of num_seqs (total is not
+// set): 1,000 of them 228.8 us, 248.7 in rows ascending.
+constexpr int kUnitChunks = 4, kUnitSeqs = 64 * kUnitChunks;
 struct UnitAt { int seq, unit, row0, rows, ctx, total; };
 __device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t* ctx_lens, int num_seqs, int UR,
                                                int i, int cols) {
+  UnitAt u{-1, 0, 0, 0, 0, 0};
+  if (num_seqs > kUnitSeqs) {
+    const int s = i % num_seqs, rank = i / num_seqs;
+    u.row0 = cu[s];
+    u.rows = cu[s + 1] - u.row0;
+    u.ctx = ctx_lens[s];
+    u.unit = (max(u.rows, 0) + UR - 1) / UR - 1 - rank;
+    if (u.unit >= 0) u.seq = s;
+    return u;
+  }
   const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
-  int c_loaded = -1, row0 = 0, rows = 0, ctx = 0, base = 0, n = 0;
-  auto load = [&](int c) {  // the sequences of chunk c, one per lane
-    if (c == c_loaded) return;
-    c_loaded = c;
+  int row0[kUnitChunks], rows[kUnitChunks], ctx[kUnitChunks], base[kUnitChunks], n[kUnitChunks];
+#pragma unroll
+  for (int c = 0; c < kUnitChunks; ++c) {  // lane l holds sequences 64 c + l
     const int s = c * 64 + lane;
-    row0 = rows = ctx = base = n = 0;
-    if (s < num_seqs) {
-      row0 = cu[s];
-      rows = cu[s + 1] - row0;
-      ctx = ctx_lens[s];
-      n = rows > 0 ? (rows + UR - 1) / UR : 0;
-      base = max(ctx - rows, 0) / UR;
+    row0[c] = rows[c] = ctx[c] = 0;
+    if (c * 64 < num_seqs && s < num_seqs) {
+      row0[c] = cu[s];
+      rows[c] = cu[s + 1] - row0[c];
+      ctx[c] = ctx_lens[s];
     }
-  };
-  const int chunks = (num_seqs + 63) / 64;
-  auto sum = [](int v) { return __builtin_amdgcn_readlane(wave_prefix_sum(v), 63); };
+  }
+#pragma unroll
+  for (int c = 0; c < kUnitChunks; ++c) {
+    n[c] = rows[c] > 0 ? (rows[c] + UR - 1) / UR : 0;
+    base[c] = max(ctx[c] - rows[c], 0) / UR;
+  }
   auto count = [&](int k) {  // units whose key is at least k
     int t = 0;
-    for (int c = 0; c < chunks; ++c) {
-      load(c);
-      t += sum(min(max(base + n - k, 0), n));
-    }
-    return t;
+#pragma unroll
+    for (int c = 0; c < kUnitChunks; ++c) t += min(max(base[c] + n[c] - k, 0), n[c]);
+    return __builtin_amdgcn_readlane(wave_prefix_sum(t), 63);
   };
-  UnitAt u{-1, 0, 0, 0, 0, 0};
   const int total = u.total = count(0);
   if (i >= cols && i < 2 * cols) i = 3 * cols - 1 - i;
   if (i >= total) return u;
   int lo = 0, hi = 0;
-  for (int c = 0; c < chunks; ++c) {
-    load(c);
-    hi = max(hi, n > 0 ? base + n - 1 : 0);
-  }
+#pragma unroll
+  for (int c = 0; c < kUnitChunks; ++c) hi = max(hi, n[c] > 0 ? base[c] + n[c] - 1 : 0);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) hi = max(hi, __shfl_xor(hi, o, 64));
   hi = __builtin_amdgcn_readfirstlane(hi);
@@ -327,20 +338,19 @@ __device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t*
     else hi = mid - 1;
   }
   int r = i - count(lo + 1);
-  for (int c = 0; c < chunks; ++c) {
-    load(c);
-    const bool has = lo >= base && lo < base + n;
+#pragma unroll
+  for (int c = 0; c < kUnitChunks; ++c) {
+    const bool has = lo >= base[c] && lo < base[c] + n[c];
     const uint64_t m = __ballot(has);
     const int here = __popcll(m);
-    if (r < here) {
+    if (u.seq < 0 && r < here) {
       const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
       const int l = __builtin_ctzll(__ballot(has && before == r));
       u.seq = c * 64 + l;
-      u.unit = lo - __builtin_amdgcn_readlane(base, l);
-      u.row0 = __builtin_amdgcn_readlane(row0, l);
-      u.rows = __builtin_amdgcn_readlane(rows, l);
-      u.ctx = __builtin_amdgcn_readlane(ctx, l);
-      return u;
+      u.unit = lo - __builtin_amdgcn_readlane(base[c], l);
+      u.row0 = __builtin_amdgcn_readlane(row0[c], l);
+      u.rows = __builtin_amdgcn_readlane(rows[c], l);
+      u.ctx = __builtin_amdgcn_readlane(ctx[c], l);
     }
     r -= here;
   }
@@ -1551,7 +1561,7 @@ extern "C" int rg_prefill_packed(const void* query, const void* key_cache, const
     // 8 heads of 128 14.2 -> 13.35, 16 of up to 64 at 28 / 4 15.0 -> 14.05, one of 500 at 32 / 8 heads
     // of 64 14.4 -> 14.05).  Not at head_dim 128 with four heads per workgroup over long tables: its
     // tile loop there is 1.3 % slower (one prompt of 2,000 tokens 41.0 against 41.6).
-    const bool direct = items <= 2 * device_cu_count() / ngroups && head_dim <= 128 &&
+    const bool direct = items <= 2 * device_cu_count() / ngroups && head_dim <= 128 && num_seqs <= kUnitSeqs &&
                         (head_dim == 64 || GW < 4 || (int64_t)max_blocks_per_seq * block_size <= 512);
     // Columns: every CU holds three workgroups of one head group (workgroup b shares its CU with
     // b +- cu_count, measured), i.e. the group's workgroups q, q + C, q + 2C with C = cu / groups.
@@ -1602,8 +1612,12 @@ extern "C" int rg_prefill_packed(const void* query, const void* key_cache, const
     const int64_t qmax = std::min<int64_t>(std::max<int32_t>(max_query_len, 1), num_tokens);
     const int64_t groups = num_heads / GW, cus = device_cu_count();
     if (cus % groups == 0 && head_dim <= 128) a.sched_cols = (int32_t)(cus / groups);  // (256: one workgroup per CU)
-    const int64_t items = (qmax + UR - 1) / UR * num_seqs, cols = std::max(a.sched_cols, 1);
-    const dim3 grid((unsigned)groups, (unsigned)std::min<int64_t>(ceil_div(items, cols) * cols, 65535));
+    const int64_t units = (qmax + UR - 1) / UR, items = units * num_seqs, cols = std::max(a.sched_cols, 1);
+    // Past kUnitSeqs a workgroup keeps to one sequence (unit_by_work): a multiple of num_seqs.
+    const int64_t wgs = num_seqs > kUnitSeqs
+                            ? num_seqs * std::max<int64_t>(1, std::min<int64_t>(units, 65535 / num_seqs))
+                            : std::min<int64_t>(ceil_div(items, cols) * cols, 65535);
+    const dim3 grid((unsigned)groups, (unsigned)wgs);
     auto go = [&](auto dtag, auto gtag) {
       constexpr int D = decltype(dtag)::value;
       constexpr int W = decltype(gtag)::value;

@@ -255,6 +255,20 @@ def test_prefill_f32_units_by_work(device, kernels, nseq, H, Hkv, D, max_query_l
 
 
 @pytest.mark.parametrize("max_query_len", [None, 1])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("nseq", [255, 256, 257, 300])
+def test_prefill_many_sequences(device, kernels, nseq, dt, max_query_len):
+    """At and past the sequences that the search by work holds (256): one unit's rows and up to
+    three, sequences without rows, an understated max_query_len, one head group."""
+    rng = np.random.default_rng(nseq)
+    lens = rng.integers(1, 20, nseq).astype(np.int32)
+    lens[2::7], lens[3::50] = 0, 70
+    prior = np.where(rng.random(nseq) < 0.5, rng.integers(1, 90, nseq), 0)
+    _run(device, kernels, _gqa_workload(4, 64, lens, prior, seed=nseq, dt=dt, H=4), seed=nseq,
+         max_query_len=max_query_len)
+
+
+@pytest.mark.parametrize("max_query_len", [None, 1])
 @pytest.mark.parametrize("dt,G,D,lens,prior", [
     ("bf16", 4, 128, [33, 1, 0, 150, 97], [0, 40, 7, 0, 300]),     # tables up to 512 tokens
     ("f16", 3, 128, [33, 1, 0, 150, 97], [0, 40, 7, 0, 1300]),
