@@ -275,9 +275,10 @@ template <> __device__ __forceinline__ float pair_sum<f16_t>(uint32_t pair, floa
 // The i-th of a batch's units of UR rows, most keys first: unit u of a sequence whose first new row
 // sits at position `first` has the work key floor(max(first, 0) / UR) + u, so a key occurs at most
 // once per sequence, and the units of at least a given key are counted with one sum over the
-// sequences, kUnitChunks to a lane and all loaded at once: a binary search over the keys, then the
-// sequences of the key found in order.  Returned wave-uniform; seq = -1 past the last unit; total
-// is their number.
+// sequences, one to a lane up to 64 of them (64 fp32 prompts 20.7 us, 22.2 with four to a lane) and
+// kUnitChunks past that, all loaded at once: a binary search over the keys, then the sequences of
+// the key found in order.  Returned wave-uniform; seq = -1 past the last unit; total is their
+// number.
 // With cols > 0 the first 2 cols units start at once and workgroups i and i + cols share a CU: the
 // second cols units are dealt in reverse, so that the longest of them go with the shortest of the
 // first.
@@ -288,22 +289,14 @@ template <> __device__ __forceinline__ float pair_sum<f16_t>(uint32_t pair, floa
 // set): 1,000 of them 228.8 us, 248.7 in rows ascending.
 constexpr int kUnitChunks = 4, kUnitSeqs = 64 * kUnitChunks;
 struct UnitAt { int seq, unit, row0, rows, ctx, total; };
-__device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t* ctx_lens, int num_seqs, int UR,
-                                               int i, int cols) {
+template <int CHUNKS>
+__device__ __forceinline__ UnitAt unit_search(const int32_t* cu, const int32_t* ctx_lens, int num_seqs, int UR,
+                                              int i, int cols) {
   UnitAt u{-1, 0, 0, 0, 0, 0};
-  if (num_seqs > kUnitSeqs) {
-    const int s = i % num_seqs, rank = i / num_seqs;
-    u.row0 = cu[s];
-    u.rows = cu[s + 1] - u.row0;
-    u.ctx = ctx_lens[s];
-    u.unit = (max(u.rows, 0) + UR - 1) / UR - 1 - rank;
-    if (u.unit >= 0) u.seq = s;
-    return u;
-  }
   const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
-  int row0[kUnitChunks], rows[kUnitChunks], ctx[kUnitChunks], base[kUnitChunks], n[kUnitChunks];
+  int row0[CHUNKS], rows[CHUNKS], ctx[CHUNKS], base[CHUNKS], n[CHUNKS];
 #pragma unroll
-  for (int c = 0; c < kUnitChunks; ++c) {  // lane l holds sequences 64 c + l
+  for (int c = 0; c < CHUNKS; ++c) {  // lane l holds sequences 64 c + l
     const int s = c * 64 + lane;
     row0[c] = rows[c] = ctx[c] = 0;
     if (c * 64 < num_seqs && s < num_seqs) {
@@ -313,14 +306,14 @@ __device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t*
     }
   }
 #pragma unroll
-  for (int c = 0; c < kUnitChunks; ++c) {
+  for (int c = 0; c < CHUNKS; ++c) {
     n[c] = rows[c] > 0 ? (rows[c] + UR - 1) / UR : 0;
     base[c] = max(ctx[c] - rows[c], 0) / UR;
   }
   auto count = [&](int k) {  // units whose key is at least k
     int t = 0;
 #pragma unroll
-    for (int c = 0; c < kUnitChunks; ++c) t += min(max(base[c] + n[c] - k, 0), n[c]);
+    for (int c = 0; c < CHUNKS; ++c) t += min(max(base[c] + n[c] - k, 0), n[c]);
     return __builtin_amdgcn_readlane(wave_prefix_sum(t), 63);
   };
   const int total = u.total = count(0);
@@ -328,7 +321,7 @@ __device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t*
   if (i >= total) return u;
   int lo = 0, hi = 0;
 #pragma unroll
-  for (int c = 0; c < kUnitChunks; ++c) hi = max(hi, n[c] > 0 ? base[c] + n[c] - 1 : 0);
+  for (int c = 0; c < CHUNKS; ++c) hi = max(hi, n[c] > 0 ? base[c] + n[c] - 1 : 0);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) hi = max(hi, __shfl_xor(hi, o, 64));
   hi = __builtin_amdgcn_readfirstlane(hi);
@@ -339,7 +332,7 @@ __device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t*
   }
   int r = i - count(lo + 1);
 #pragma unroll
-  for (int c = 0; c < kUnitChunks; ++c) {
+  for (int c = 0; c < CHUNKS; ++c) {
     const bool has = lo >= base[c] && lo < base[c] + n[c];
     const uint64_t m = __ballot(has);
     const int here = __popcll(m);
@@ -354,6 +347,20 @@ __device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t*
     }
     r -= here;
   }
+  return u;
+}
+
+__device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t* ctx_lens, int num_seqs, int UR,
+                                               int i, int cols) {
+  if (num_seqs <= 64) return unit_search<1>(cu, ctx_lens, num_seqs, UR, i, cols);
+  if (num_seqs <= kUnitSeqs) return unit_search<kUnitChunks>(cu, ctx_lens, num_seqs, UR, i, cols);
+  UnitAt u{-1, 0, 0, 0, 0, 0};
+  const int s = i % num_seqs, rank = i / num_seqs;
+  u.row0 = cu[s];
+  u.rows = cu[s + 1] - u.row0;
+  u.ctx = ctx_lens[s];
+  u.unit = (max(u.rows, 0) + UR - 1) / UR - 1 - rank;
+  if (u.unit >= 0) u.seq = s;
   return u;
 }
 
