@@ -257,7 +257,7 @@ def test_prefill_f32_units_by_work(device, kernels, nseq, H, Hkv, D, max_query_l
 @pytest.mark.parametrize("max_query_len", [None, 1])
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("nseq", [255, 256, 257, 300])
-def test_prefill_many_sequences(device, kernels, nseq, dt, max_query_len):
+def test_prefill_many_sequences_by_work(device, kernels, nseq, dt, max_query_len):
     """At and past the sequences that the search by work holds (256): one unit's rows and up to
     three, sequences without rows, an understated max_query_len, one head group."""
     rng = np.random.default_rng(nseq)

@@ -240,3 +240,18 @@ def test_deinterleave_gate_up_inverts_the_layout():
     assert torch.equal(deinterleave_gate_up(il.t()).t(), w)
     x = torch.randn(rows, k, generator=g)
     assert torch.equal(deinterleave_gate_up(x @ il.t()), x @ w.t())
+
+
+def test_no_test_function_is_defined_twice():
+    """A second function of the same name replaces the first one when its module is loaded, whose
+    cases are then collected no more."""
+    import ast
+    from collections import Counter
+
+    here = os.path.join(ROOT, "tests")
+    for name in sorted(os.listdir(here)):
+        if name.startswith("test_") and name.endswith(".py"):
+            tree = ast.parse(open(os.path.join(here, name)).read())
+            for scope in [tree] + [n for n in tree.body if isinstance(n, ast.ClassDef)]:
+                count = Counter(n.name for n in scope.body if isinstance(n, ast.FunctionDef))
+                assert [n for n, c in count.items() if c > 1] == [], name
