@@ -26,6 +26,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "gemm_plan.hpp"
 #include "rg_common.hpp"
 
 namespace rg {
@@ -48,12 +49,6 @@ template <> struct gemm_mfma<f16_t> {
                                                   __builtin_bit_cast(gf16x8_t, b), c, 0, 0, 0);
   }
 };
-
-constexpr int kGemmWaves = 4;
-constexpr int kGemmMaxRows = 128;
-#ifndef RG_GEMM_AHEAD
-#define RG_GEMM_AHEAD 2
-#endif
 
 struct GemmArgs {
   const uint16_t* x;
@@ -93,10 +88,6 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x70 | 0xF00);
 }
 
-// Chunks of 128 k: 256 bytes of every row of X and W.
-constexpr int kChunkK = 128;
-constexpr int kChunkBytes = 2 * kChunkK;
-constexpr int kLdsBytes = 160 * 1024;
 constexpr int kGemmThreads = 64 * kGemmWaves;
 
 // LDS ring of one instantiation: a slot holds a chunk of X (16 MB rows) then of W (16 NB rows).
@@ -147,8 +138,6 @@ constexpr int kEpiPlain = 0;
 constexpr int kEpiSiluMul = 1;
 constexpr int kEpiRope = 2;
 constexpr int kEpiResidual = 3;  // C[m][n] <- round(C[m][n] + round(X . W^T)): the residual add
-// Largest K of the NORM kernels (their norm weight is staged whole in LDS).
-constexpr int kNormMaxK = 8192;
 
 // The 8 values of a 16-byte fragment as floats.
 template <typename T>
@@ -657,71 +646,6 @@ void launch_gemm_rope(const GemmArgs& a, int nb, int mb, hipStream_t s) {
   else launch_gemm_mb<T, 2, kEpiRope, NORM>(a, mb, 1, s);
 }
 
-// Chunks in flight and LDS bytes of a workgroup of the (NB, MB) instantiation (GemmRing<NB, MB,
-// reserve>::AHEAD and ::BYTES + reserve, the norm weight's bytes of the NORM kernels).
-int ring_ahead(int nb, int mb, int reserve = 0) {
-  const int fit = (kLdsBytes - reserve) / (16 * (mb + nb) * kChunkBytes);
-  return fit >= RG_GEMM_AHEAD + 2 ? RG_GEMM_AHEAD : fit >= 3 ? fit - 2 : fit - 1;
-}
-int ring_bytes(int nb, int mb, int reserve = 0) {
-  const int slot = 16 * (mb + nb) * kChunkBytes;
-  const int fit = (kLdsBytes - reserve) / slot;
-  const int ahead = ring_ahead(nb, mb, reserve);
-  const int slots = fit >= ahead + 2 ? ahead + 2 : ahead + 1;
-  return std::max(slots * slot, nb * mb * kGemmWaves * 1024) + reserve;
-}
-
-// Workgroup shape: 16-column n-blocks (NB) and 16-row blocks (MB) per workgroup, row tiles
-// ceil(M / 16 MB) and splits of K, chosen by a cost model of the per-CU operand stream
-// calibrated on MI355X (a sweep of every shape at 1 to 128 rows of the projections of three model
-// sizes, weights cold):
-//   workgroups = row tiles x column tiles x splits, R = CUs x resident workgroups per CU (LDS),
-//   stream = 3 us x ceil(workgroups / R) + 0.047 us x ceil(workgroups / CUs) x (MB + NB) x chunks / S
-//            (0.047 us per 16 rows x 128 k: 4 KB of copies),
-//   turn = 3 us + 0.18 us x sqrt(2 / chunks in flight) x chunks / S: a workgroup walks its chunks one
-//          after the other, a copy's round trip over the chunks in flight each, however few bytes
-//          they hold (4096 x 14336 unsplit, 112 chunks in turn, took 30 us whatever its rows),
-//   serial = max(stream, ceil(workgroups / R) x turn), weights = N K 2 B / 5.5 TB/s,
-//   time = max(serial, weights) + 0.2 min(serial, weights) + 0.1 stream + (S > 1: 2 us + S M N 8 B /
-//          3 TB/s for the partials and their reduce).
-// Without the turn the model left deep layers unsplit: 4096 x 14336 at 1 / 27 / 64 rows 30.5 / 33.2
-// / 36.7 us against 22.1 / 22.9 / 31.8 now (the weights alone 18.9 at 6.2 TB/s), 3072 x 8192 at 1
-// to 16 rows 17.8 against 13.5.  Over that sweep its pick is 1.6 % from the measured best on average
-// (7.9 % without) and nowhere slower than before.
-// Each workgroup streams its rows of X and its columns of W once per K range; small row tiles
-// cut the X bytes of narrow layers, and the XCD-aware order keeps their re-reads of W in L2.
-struct GemmPlan { int nb, mb, mtiles, splits, xcd; };
-GemmPlan gemm_plan(int M, int N, int K, int cus, bool pairs = false, int only_nb = 0, bool norm = false) {
-  const int nblk = N / 16, chunks = K / kChunkK;
-  GemmPlan best{1, 1, M, 1, 0};
-  double best_t = 1e30;
-  for (int mb : {1, 2, 4, 8}) {
-    if (mb > 1 && 16 * (mb / 2) >= M) continue;  // a smaller row tile already holds every row
-    const int mtiles = (M + 16 * mb - 1) / (16 * mb);
-    for (int nb : {4, 2, 1}) {
-      if (nblk % nb != 0 || (pairs && nb == 1) || (only_nb && nb != only_nb)) continue;
-      const int resident = std::max(1, std::min(4, kLdsBytes / ring_bytes(nb, mb, norm ? 2 * kNormMaxK : 0)));
-      for (int splits : {1, 2, 4}) {
-        if (splits > 1 && (pairs || norm || chunks / splits < 8)) continue;
-        const int64_t wgs = (int64_t)mtiles * (nblk / nb) * splits;
-        const double stream = 3.0 * (double)ceil_div(wgs, (int64_t)cus * resident) +
-                              0.047 * (double)ceil_div(wgs, cus) * (mb + nb) * (chunks / splits);
-        const int ahead = ring_ahead(nb, mb, norm ? 2 * kNormMaxK : 0);
-        const double turn = 3.0 + 0.18 * std::sqrt(2.0 / ahead) * chunks / splits;
-        const double serial = std::max(stream, (double)ceil_div(wgs, (int64_t)cus * resident) * turn);
-        const double weights = (double)N * K * 2 / 5.5e6;
-        double t = std::max(serial, weights) + 0.2 * std::min(serial, weights) + 0.1 * stream;
-        if (splits > 1) t += 2.0 + (double)splits * M * N * 8 / 3.0e6;
-        if (t < best_t - 1e-9) {
-          best_t = t;
-          best = GemmPlan{nb, mb, mtiles, splits, mtiles > 1 && (nblk / nb) % 8 == 0 ? 1 : 0};
-        }
-      }
-    }
-  }
-  return best;
-}
-
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
@@ -735,8 +659,7 @@ extern "C" size_t rg_linear_workspace_bytes(int32_t num_rows, int32_t out_featur
     return 0;
   }
   if (wide_fits(num_rows, out_features, in_features, in_features)) return 0;  // the wide form: one pass
-  const GemmPlan p = gemm_plan(num_rows, out_features, in_features, device_cu_count());
-  return p.splits > 1 ? (size_t)p.splits * num_rows * out_features * sizeof(float) : 0;
+  return split_bytes(gemm_plan(num_rows, out_features, in_features, device_cu_count()), num_rows, out_features);
 }
 
 namespace rg {
@@ -787,11 +710,8 @@ int linear_entry(const char* op, const void* x, const void* weight, void* out, i
   bool empty = false;
   if (int st = check_linear(op, x, weight, out, M, N, K, N, ldx, ldw, ldo, dtype, empty)) return st;
   if (empty) return ok();
-  GemmPlan plan = gemm_plan(M, N, K, device_cu_count());
-  const size_t need = plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
-  if (need > 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))) {
-    plan.splits = 1;  // no (or too small a) workspace: one pass over K
-  }
+  const GemmPlan plan =
+      linear_plan(M, N, K, device_cu_count(), workspace != nullptr && aligned16(workspace) ? workspace_bytes : 0);
   GemmArgs a{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(weight), static_cast<uint16_t*>(out),
              static_cast<float*>(workspace), M, N, K, ldx, ldw, ldo, plan.mtiles, plan.xcd};
   a.stagger = stagger_for(N, K);

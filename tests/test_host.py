@@ -255,3 +255,39 @@ def test_no_test_function_is_defined_twice():
             for scope in [tree] + [n for n in tree.body if isinstance(n, ast.ClassDef)]:
                 count = Counter(n.name for n in scope.body if isinstance(n, ast.FunctionDef))
                 assert [n for n, c in count.items() if c > 1] == [], name
+
+
+def test_gemm_plan_without_room_to_split(tmp_path):
+    """A projection whose workspace does not hold the partials of the best plan runs on the best plan
+    with fewer splits (unsplit without any), not on the split plan's few wide tiles: gemm_plan.hpp on
+    a 256-CU device, rows from one to the limit, deep, wide and narrow layers."""
+    src, exe = tmp_path / "plan.cpp", tmp_path / "plan"
+    src.write_text("""
+#include <cstdio>
+#include "gemm_plan.hpp"
+using namespace rg;
+int main() {
+  for (auto [N, K] : {std::pair{4096, 14336}, {3072, 8192}, {2048, 8192}, {4096, 4096}, {1024, 4096}, {16384, 2048}, {16, 128}})
+    for (int M : {1, 5, 16, 17, 27, 33, 64, 65, 128}) {
+      const size_t need = split_bytes(gemm_plan(M, N, K, 256), M, N);
+      for (size_t ws : {(size_t)0, need ? need - 1 : 0, need}) {
+        const GemmPlan p = linear_plan(M, N, K, 256, ws), u = gemm_plan(M, N, K, 256, false, 0, false, 1);
+        printf("%d %d %d %zu %zu %d %d %d %d %d\\n", M, N, K, need, ws, p.nb, p.mb, p.splits, u.nb, u.mb);
+      }
+    }
+}
+""")
+    csrc = os.path.join(ROOT, "railgun_amd", "csrc")
+    subprocess.run(["g++", "-std=c++20", "-Wall", "-Werror", f"-I{csrc}", str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+    split = 0
+    for line in out.splitlines():
+        M, N, K, need, ws, nb, mb, splits, u_nb, u_mb = map(int, line.split())
+        assert splits * M * N * 4 <= ws or splits == 1, line
+        assert splits > 1 or need == 0 or (nb, mb) == (u_nb, u_mb), line
+        if ws == need:
+            assert (splits > 1) == (need > 0) and splits * M * N * 4 == max(need, splits * M * N * 4), line
+            split += splits > 1
+        if (M, N, K, ws) == (64, 4096, 14336, 0):
+            assert (N // (16 * nb)) * -(-M // (16 * mb)) >= 256, line  # (64 of the split plan's tiles)
+    assert split >= 20
