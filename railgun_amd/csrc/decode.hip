@@ -1472,15 +1472,15 @@ __global__ __launch_bounds__(64 * G) void decode_stream_merge_kernel(StreamArgs 
 //
 // Tables of few tokens (short_applies): one workgroup per segment (sequence, kv-head), kShortWaves
 // waves taking its 16-token sub-blocks in turn, their partials merged in LDS and the output written:
-// one launch and no scratch.  Such a call is bound by latency and launches, not by bytes: the
+// one launch, and the workspace, whose size is asked for by shape alone, is left alone.  Such a call is bound by latency and launches, not by bytes: the
 // stream-K worker first finds its range by a scan over the context lengths, then its block-table
 // window, then its K/V rows, and the merge kernel follows.  Here the table entries (lane l of wave w
 // holds sub-block w + kShortWaves l), the context length and q are loaded at once, then the K/V
 // rows.  ROPE as in decode_stream_kernel: every wave rotates its q rows, the wave holding the last
 // sub-block writes and patches the new token's rows.
 // Measured (kernel trace, 4 sequences): 32 / 8 heads of 128 in bf16 at 100 tokens 7.8 us against 9.5 +
-// 3.4 of the two kernels and the gap between them, 11.3 against 8.9 + 3.8 at 400; fp32 heads of 64 at
-// 400 tokens 10.4 against 8.8 + 3.4.  Its slope is P.V on the VALU, ~1,100 cycles a sub-block and
+// 3.4 of the two kernels and the gap between them; fp32 heads of 64 at 400 tokens 10.4 against 8.8 +
+// 3.4.  Its slope is P.V on the VALU, ~1,100 cycles a sub-block and
 // wave; 16 tokens a wave more cost 1.1 us.
 constexpr int kShortWaves = 8;
 constexpr int kShortThreads = 64 * kShortWaves;
@@ -1986,23 +1986,22 @@ size_t stream_bytes(const Shape& sh, int32_t workers, StreamScratch* carve, void
   return acc + ml + desc;
 }
 
-// Whether the one-launch kernel takes the call: G 1 to 8 at head_dim 64 or 128, at most 256 KB of K
-// and V in a segment's table row (one CU streams a segment at ~41 GB/s here; at 400 KB the two
-// kernels together are as fast on the device, and at 800 KB 5 us faster) and at most 64 MB in the
-// whole table (64 sequences of 400 tokens at 8 kv-heads of 128, 105 MB: 32.6 us a pass of RoPE and
-// decode against 26.5; 16 of 800, 52 MB: 23.8 against 26.1).  The table's width stands for the
-// contexts, which the host does not know: contexts shorter than it only make the call shorter.
-#ifndef RG_SHORT_KB
-#define RG_SHORT_KB 256
-#endif
-#ifndef RG_SHORT_TOTAL_MB
-#define RG_SHORT_TOTAL_MB 64
-#endif
+// Whether the one-launch kernel takes the call: G 1 to 8 at head_dim 64 or 128, and the lines below
+// on the table's width, which stands for the contexts that the host does not know (contexts shorter
+// than it only make the call shorter), and on the segments.  One CU streams a segment, and a second
+// workgroup does not fit beside the first, so the segments past one per CU run after the others.
+//   Up to one segment per CU: the last width at which no ratio of heads (1, 4, 7, 8) at 8 to 256
+// segments was slower than the two kernels back to back (time here over time there, mean and worst):
+// head_dim 128 in 16 bits 0.90 / 0.96 at 320 tokens, 0.96 / 1.05 at 384, 1.08 / 1.19 at 512; in
+// fp32 0.88 / 0.92 at 192, 0.97 / 1.08 at 256; head_dim 64 in 16 bits 0.89 / 1.00 at 896, 0.95 / 1.06
+// at 1,024; in fp32 0.92 / 0.98 at 512.
+//   Up to two per CU: 64 tokens, 0.92 at worst (264 to 512 segments); at 128 already 1.33, at 320
+// 1.48.  More: never (1,024 segments of 64 tokens 1.27 to 1.60).
 bool short_applies(const Shape& sh, int elem_bytes) {
-  const int64_t tokens = (int64_t)sh.MB * sh.bs, segment = tokens * sh.D * 2 * elem_bytes;
-  return (sh.D == 64 || sh.D == 128) && sh.H / sh.Hkv <= 8 && tokens <= kShortMaxTokens &&
-         segment <= (int64_t)RG_SHORT_KB << 10 && segment * sh.B * sh.Hkv <= (int64_t)RG_SHORT_TOTAL_MB << 20 &&
-         sh.B <= 65535;
+  const int64_t tokens = (int64_t)sh.MB * sh.bs, segments = (int64_t)sh.B * sh.Hkv, cus = device_cu_count();
+  const int64_t widest = (sh.D == 64 ? 224 : 160) + (elem_bytes == 4 ? 32 : 0);  // KB of K and V
+  return (sh.D == 64 || sh.D == 128) && sh.H / sh.Hkv <= 8 && tokens <= kShortMaxTokens && sh.B <= 65535 &&
+         (segments <= cus ? tokens * sh.D * 2 * elem_bytes <= widest << 10 : segments <= 2 * cus && tokens <= 64);
 }
 
 template <typename T, int D, int G, bool ROPE = false>

@@ -609,8 +609,10 @@ SHORT_EDGES = [0, 1, 15, 16, 17, 127, 128, 129, 255, 256, 257]  # sub-block and 
 
 
 @pytest.mark.parametrize("dt,D,bs,mb", [
-    ("bf16", 128, 16, 32), ("bf16", 128, 16, 33),   # 256 KB of K/V per segment: the one-launch kernel; past it
-    ("f16", 64, 32, 32), ("f16", 64, 32, 33), ("f32", 64, 16, 32), ("f32", 128, 16, 16), ("f32", 128, 64, 4)])
+    ("bf16", 128, 16, 20), ("bf16", 128, 16, 21),   # the widest table of the one-launch kernel; past it
+    ("bf16", 128, 16, 32), ("bf16", 128, 16, 33), ("f16", 64, 32, 28), ("f16", 64, 32, 29), ("f16", 64, 32, 32),
+    ("f16", 64, 32, 33), ("f32", 64, 16, 32), ("f32", 64, 16, 33), ("f32", 128, 16, 12), ("f32", 128, 16, 13),
+    ("f32", 128, 16, 16), ("f32", 128, 64, 3), ("f32", 128, 64, 4)])
 @pytest.mark.parametrize("G", [1, 3, 4, 8])
 def test_decode_short_tables(device, kernels, dt, D, bs, mb, G):
     """Tables of few tokens (decode_short_kernel) at the edges of its waves' turns, up to the whole
@@ -623,9 +625,41 @@ def test_decode_short_tables(device, kernels, dt, D, bs, mb, G):
     np.testing.assert_array_equal(got[0], 0)
 
 
+def _in_one_launch(device, kernels, inp) -> bool:
+    """Whether v1 left its workspace alone, after a check of its output."""
+    B, shape = len(inp["ctx"]), (inp["H"], inp["Hkv"], inp["D"], inp["bs"], inp["mb"])
+    ws = torch.full((kernels.v1_workspace_bytes(B, *shape),), 0xA5, dtype=torch.uint8, device=device)
+    out = torch.full_like(inp["dq"], float("nan"))
+    kernels.launch_v1(inp["dq"], inp["dkc"], inp["dvc"], inp["dbt"], inp["dctx"], out, inp["scale"], *shape, B,
+                      workspace=ws)
+    torch.cuda.synchronize()
+    assert_close(dev_f32(out), oracle_v1_plus(inp), inp["dt"])
+    return bool((ws == 0xA5).all())
+
+
+@pytest.mark.parametrize("dt,D,widest", [("bf16", 128, 320), ("f16", 64, 896), ("f32", 128, 192), ("f32", 64, 512)])
+@pytest.mark.parametrize("G", [1, 8])
+def test_decode_short_tables_line(device, kernels, dt, D, widest, G):
+    """The one-launch kernel ends where the two kernels become faster: it takes the widest table of
+    the line and none wider.  The route shows in the workspace, which only the two kernels write."""
+    for tokens, one_launch in ((widest, True), (widest + 16, False)):
+        inp = make_inputs(device, [tokens, 17], dt, H=2 * G, Hkv=2, D=D, seed=tokens + G, mb=tokens // 16)
+        assert _in_one_launch(device, kernels, inp) == one_launch, f"{tokens} tokens"
+
+
+@pytest.mark.parametrize("batch,tokens,one_launch", [(32, 320, True), (33, 80, False), (33, 64, True), (64, 64, True),
+                                                     (65, 64, False), (64, 80, False)])
+def test_decode_short_tables_segments(device, kernels, batch, tokens, one_launch):
+    """One segment per CU takes the whole line's width, up to two per CU 64 tokens, more none (8
+    kv-heads; 256 CUs)."""
+    ctx = [tokens] + [1 + (7 * s) % tokens for s in range(1, batch)]
+    inp = make_inputs(device, ctx, "bf16", H=16, Hkv=8, D=128, seed=batch, mb=tokens // 16)
+    assert _in_one_launch(device, kernels, inp) == one_launch
+
+
 @pytest.mark.parametrize("batch", [64, 65])
 def test_decode_short_tables_total(device, kernels, batch):
-    """At and past 64 MB of K/V in the whole table (8 kv-heads of 64 in fp32, 256 tokens each)."""
+    """Around 64 MB of K/V in tables of 256 tokens, two segments per CU (8 kv-heads of 64 in fp32)."""
     rng = np.random.default_rng(batch)
     inp = make_inputs(device, rng.integers(0, 257, batch), "f32", H=16, Hkv=8, D=64, seed=batch, mb=16)
     assert_close(gpu_v1(kernels, inp, workspace=True), oracle_v1_plus(inp), "f32", f"batch {batch}")
