@@ -1180,7 +1180,8 @@ __global__ __launch_bounds__(kPThreads, DIRECT ? 2 : pf_wg_per_cu<D>()) void pre
 //    every copy) the 5 prompts above took 146 us, 113 with it (75 TFLOP/s, 49 % of what a large
 //    fp32 product reaches here); 12 prompts of 128 to 2,048 tokens at head_dim 128 2,158 -> 1,749
 //    us a call with the cache write, 6 of up to 700 behind up to 500 cached at head_dim 256 529 ->
-//    304.  The arithmetic and its order are unchanged.
+//    304.  The arithmetic and its order are those of softmax and PV in turn; new_maximum below says
+//    how the probabilities keep their subnormal values.
 //
 //  * Scores transposed, S^T = K Q^T: lane (row l % 32, half h = l / 32) provides K[key l % 32]
 //    and Q[query l % 32] at the d of MFMA k-index h; inside a pair of steps the d order is
@@ -1225,7 +1226,8 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
   int key_cap = a.max_blocks * bs;  // positions the table row can address
 
   for (int i = blockIdx.y;; i += gridDim.y) {
-    const UnitAt at = unit_by_work(a.cu_seqlens, a.context_lens, a.num_seqs, UR, i, a.sched_cols);
+    const UnitAt at =
+        unit_by_work(a.cu_seqlens, a.context_lens, a.num_seqs, UR, i, D > 128 ? 0 : a.sched_cols);
     if (at.seq < 0) break;
     const int unit = at.unit, row0 = at.row0, L = at.rows, ctx = at.ctx;
     const int first = ctx - L;           // position of the sequence's first new row
@@ -1339,40 +1341,52 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
           if (!row_ok || key > qpos || key >= nkeys) st[4 * j + r] = -INFINITY;
         }
     };
-    // Online softmax (log2 units) of scores st, which become probabilities, in the parts 0 .. 11
-    // that ride along with the next tile's QK steps; rescale then applies the new maximum to o.
-    float mx = 0.f, mref = 0.f, alpha = 0.f, ps = 0.f;
-    bool moved = false;
-    auto softmax_part = [&](f32x16& st, auto part) __attribute__((always_inline)) {
+    // Online softmax (log2 units) of scores st: new_maximum, then the probabilities in place of the
+    // scores, in the parts 0 .. 7 that ride along with the next tile's QK steps; rescale then applies
+    // the new maximum to o.
+    // v_exp_f32 by itself has no subnormal results, and exp2f, which has, in its place costs 7 % of the
+    // call at head_dim 64 and 4 % at 128 (fp32 MFMAs leave the vector units no free cycles).  So the
+    // parts take the instruction, and a tile with a factor or a probability below 2^-126 (`deep`, seen
+    // by its smallest score) is done before them with exp2f, which costs 1.3 % and 0.6 %.  A row whose
+    // scores are NaN gives NaN.
+    float mref = 0.f, alpha = 0.f, ps = 0.f;
+    bool deep = false;
+    auto new_maximum = [&](const f32x16& st) __attribute__((always_inline)) {
+      float mx = st[0], least = st[0];
+#pragma unroll
+      for (int e = 1; e < 16; ++e) mx = fmaxf(mx, st[e]), least = fminf(least, st[e]);
+      const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      const float mn = fmaxf(m, fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1])));
+      // A row without a key yet keeps its maximum of -inf: 0 in its place gives exponents of
+      // -inf - 0, probabilities 0.
+      mref = mn == -INFINITY ? 0.f : mn;
+      const float drop = m - mref;
+      alpha = __builtin_amdgcn_exp2f(drop);
+      deep = __ballot(least - mref < -126.f || fabsf(drop + 138.f) < 13.f) != 0;
+      if (deep) alpha = exp2f(drop);
+      m = mn;
+      ps = 0.f;
+    };
+    auto softmax_part = [&](f32x16& st, auto part, auto exact) __attribute__((always_inline)) {
       constexpr int P = decltype(part)::value;
-      if constexpr (P == 0) {
-        mx = st[0];
+      if constexpr (P < 8) {
 #pragma unroll
-        for (int e = 1; e < 16; ++e) mx = fmaxf(mx, st[e]);
-      } else if constexpr (P == 1) {
-        ps = __shfl_xor(mx, 32, 64);
-      } else if constexpr (P == 3) {
-        const float mn = fmaxf(m, fmaxf(mx, ps));
-        // A row without a key yet keeps its maximum of -inf: 0 in its place gives exponents of
-        // -inf - 0, probabilities 0.
-        mref = mn == -INFINITY ? 0.f : mn;
-        alpha = __builtin_amdgcn_exp2f(m - mref);
-        moved = __ballot(m != mn) != 0;  // else every alpha that matters is exactly 1
-        m = mn;
-        ps = 0.f;
-      } else if constexpr (P >= 4 && P < 12) {
-#pragma unroll
-        for (int e = 2 * (P - 4); e < 2 * (P - 4) + 2; ++e) {
-          float pe = __builtin_amdgcn_exp2f(st[e] - mref);
+        for (int e = 2 * P; e < 2 * P + 2; ++e) {
+          float pe = decltype(exact)::value ? exp2f(st[e] - mref) : __builtin_amdgcn_exp2f(st[e] - mref);
           ps += pe;
           asm volatile("" : "+v"(pe));  // formed here, not behind the branch of rescale
           st[e] = pe;
         }
-        if constexpr (P == 11) lsum = lsum * alpha + ps;
+        if constexpr (P == 7) lsum = lsum * alpha + ps;
       }
     };
+    auto softmax_exact = [&](f32x16& st) __attribute__((always_inline)) {
+      [&]<int... P>(std::integer_sequence<int, P...>) __attribute__((always_inline)) {
+        (softmax_part(st, std::integral_constant<int, P>{}, std::true_type{}), ...);
+      }(std::make_integer_sequence<int, 8>{});
+    };
     auto rescale = [&]() __attribute__((always_inline)) {
-      if (moved) {
+      if (__ballot(alpha != 1.f) != 0) {  // (a maximum that stays gives exactly 1)
 #pragma unroll
         for (int b = 0; b < NDB; ++b) o[b] *= alpha;
       }
@@ -1436,7 +1450,14 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
       for (int kt = 0; kt < kfull - 1; ++kt) {
         copies(kt);
         mask(st, kt);
-        const f32x16 nx = scores(kt + 1, [&](auto c) __attribute__((always_inline)) { softmax_part(st, c); });
+        new_maximum(st);
+        f32x16 nx;
+        if (deep) {
+          softmax_exact(st);
+          nx = scores(kt + 1, [](auto) {});
+        } else {
+          nx = scores(kt + 1, [&](auto c) __attribute__((always_inline)) { softmax_part(st, c, std::false_type{}); });
+        }
         rescale();
         accumulate(st, kt);
         st = nx;
@@ -1444,9 +1465,8 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
       if (kfull > 0) {
         copies(kfull - 1);
         mask(st, kfull - 1);
-        [&]<int... P>(std::integer_sequence<int, P...>) __attribute__((always_inline)) {
-          (softmax_part(st, std::integral_constant<int, P>{}), ...);
-        }(std::make_integer_sequence<int, 12>{});
+        new_maximum(st);
+        softmax_exact(st);
         rescale();
         accumulate(st, kfull - 1);
       }

@@ -254,6 +254,63 @@ def test_prefill_f32_units_by_work(device, kernels, nseq, H, Hkv, D, max_query_l
     _run(device, kernels, w, seed=nseq + 1, max_query_len=max_query_len)
 
 
+def _run_f32_rows(device, kernels, D, q0, key0, val):
+    """One sequence of len(key0) rows at 4 / 1 heads: q row r is q0[r] and key t key0[t] in their first
+    dim (0 in the others), value t is val[t] in every dim; scale 1.  Returns the first head's dims."""
+    n = len(key0)
+    q = torch.zeros(n, 4, D, device=device)
+    q[:, :, 0] = torch.as_tensor(q0, dtype=torch.float32, device=device)[:, None]
+    kc, vc = torch.zeros(8, 16, D, device=device), torch.zeros(8, 16, D, device=device)
+    kc.view(128, D)[:n, 0] = torch.as_tensor(key0, dtype=torch.float32, device=device)
+    vc.view(128, D)[:n] = torch.as_tensor(val, dtype=torch.float32, device=device)[:, None]
+    out = torch.full_like(q, float("nan"))
+    kernels.launch_prefill_packed(q, kc.view(8, 1, 16, D), vc.view(8, 1, 16, D), i32(np.arange(8)[None], device),
+                                  i32([n], device), i32([0, n], device), out, 1.0, 4, 1, D, 16, 8, 1, n, n)
+    torch.cuda.synchronize()
+    return dev_f32(out)[:, 0]
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("case", ["probability", "rescale"])
+def test_prefill_f32_subnormal_weights(device, kernels, D, case):
+    """Probabilities and rescale factors of 2^-130, below the smallest normal fp32 number, still weigh
+    their values (here 2^100): in the first case every key but the first lies 130 below it in log2
+    units, in the second the keys from 35 on lie 130 above the first tile's.  The score carries two
+    roundings (log2 e, the product), 2 2^-24 of 130 ln 2 = 1.1e-5 of the weight, a subnormal of
+    2^-130 one of 2^-20 and the sums over 70 keys 4e-6 at most: 2e-5."""
+    n, step = 70, 130 * math.log(2)
+    key, val = np.zeros(n), np.zeros(n)
+    if case == "probability":
+        key[1:], val[1:] = -step, 2.0 ** 100
+    else:
+        key[35:], val[:32] = step, 2.0 ** 100
+    got = _run_f32_rows(device, kernels, D, np.ones(n), key, val)
+    key = key.astype(np.float32).astype(np.float64)
+    p = np.tril(np.exp(key[None] - np.maximum.accumulate(key)[:, None]))
+    want = (p @ val) / p.sum(1)
+    np.testing.assert_allclose(got, np.broadcast_to(want[:, None], got.shape), rtol=2e-5, atol=0)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_prefill_f32_nan_and_infinite_scores(device, kernels, D):
+    """A row whose scores are NaN gives NaN, as the oracle and the generic kernel do, and leaves the
+    others alone; a row that sees only scores of -inf has no weight to share and gives zeros; a
+    score of -inf beside finite ones weighs nothing."""
+    n = 70
+    key = np.linspace(-2, 2, n)
+    key[40] = -np.inf
+    q0 = np.ones(n)
+    q0[3], q0[50] = np.nan, np.nan
+    val = np.cos(np.arange(n))
+    got = _run_f32_rows(device, kernels, D, q0, key, val)
+    assert np.isnan(got[[3, 50]]).all()
+    p = np.tril(np.exp(key)[None].repeat(n, 0))
+    want = ((p @ val) / p.sum(1))[:, None]
+    rows = np.setdiff1d(np.arange(n), [3, 50])
+    np.testing.assert_allclose(got[rows], np.broadcast_to(want[rows], got[rows].shape), rtol=0, atol=2e-6)
+    np.testing.assert_array_equal(_run_f32_rows(device, kernels, D, np.ones(5), np.full(5, -np.inf), val[:5]), 0)
+
+
 @pytest.mark.parametrize("max_query_len", [None, 1])
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("nseq", [255, 256, 257, 300])
