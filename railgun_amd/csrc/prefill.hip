@@ -255,6 +255,16 @@ __device__ __forceinline__ int wave_prefix_sum(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
   return v;
 }
+// Maximum over the 64 lanes of values not below 0, in the same steps.
+__device__ __forceinline__ int wave_max(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(v, 63);
+}
 // Orders this wave's earlier LDS writes before its later LDS reads.
 __device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 constexpr int kSchedSeqs = 256;
@@ -277,18 +287,19 @@ template <> __device__ __forceinline__ float pair_sum<f16_t>(uint32_t pair, floa
 // once per sequence, and the units of at least a given key are counted with one sum over the
 // sequences, one to a lane up to 64 of them (64 fp32 prompts 20.7 us, 22.2 with four to a lane) and
 // kUnitChunks past that, all loaded at once: a binary search over the keys, then the sequences of
-// the key found in order.  Returned wave-uniform; seq = -1 past the last unit; total is their
-// number.
+// the key found in order.  Returned wave-uniform; seq = -1 for an i without a unit; no i from end on
+// has one, so a caller that steps through them stops there without another search (a wasted one at
+// the end of every workgroup cost 255 fp32 prompts of 40 rows at 32 / 32 heads of 64 a fifth of 253 us).
 // With cols > 0 the first 2 cols units start at once and workgroups i and i + cols share a CU: the
 // second cols units are dealt in reverse, so that the longest of them go with the shortest of the
 // first.
 // More than kUnitSeqs sequences would have to be read again at every step of the search, a round
 // trip each (fp32 prompts of up to 40 rows, 32 / 8 heads of 64, 64 sequences to a read: 256 of them
 // 76.5 us against 61.0 so, 1,000 562.7): no search then, item i is the (i / num_seqs)-th unit from
-// the end of sequence i % num_seqs, and the caller steps by a multiple of num_seqs (total is not
-// set): 1,000 of them 228.8 us, 248.7 in rows ascending.
+// the end of sequence i % num_seqs, and the caller steps by a multiple of num_seqs: 1,000 of them
+// 228.8 us, 248.7 in rows ascending.
 constexpr int kUnitChunks = 4, kUnitSeqs = 64 * kUnitChunks;
-struct UnitAt { int seq, unit, row0, rows, ctx, total; };
+struct UnitAt { int seq, unit, row0, rows, ctx, end; };
 template <int CHUNKS>
 __device__ __forceinline__ UnitAt unit_search(const int32_t* cu, const int32_t* ctx_lens, int num_seqs, int UR,
                                               int i, int cols) {
@@ -316,21 +327,25 @@ __device__ __forceinline__ UnitAt unit_search(const int32_t* cu, const int32_t* 
     for (int c = 0; c < CHUNKS; ++c) t += min(max(base[c] + n[c] - k, 0), n[c]);
     return __builtin_amdgcn_readlane(wave_prefix_sum(t), 63);
   };
-  const int total = u.total = count(0);
+  const int total = count(0);
+  u.end = total > cols ? max(total, 2 * cols) : total;  // (of the reversed ones any may have a unit)
   if (i >= cols && i < 2 * cols) i = 3 * cols - 1 - i;
   if (i >= total) return u;
   int lo = 0, hi = 0;
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) hi = max(hi, n[c] > 0 ? base[c] + n[c] - 1 : 0);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) hi = max(hi, __shfl_xor(hi, o, 64));
-  hi = __builtin_amdgcn_readfirstlane(hi);
+  hi = wave_max(hi);
+  int above = 0;     // units at or above key hi + 1
   while (lo < hi) {  // the largest key with more than i units at or above it
-    const int mid = (lo + hi + 1) >> 1;
-    if (count(mid) > i) lo = mid;
-    else hi = mid - 1;
+    const int mid = (lo + hi + 1) >> 1, c = count(mid);
+    if (c > i) {
+      lo = mid;
+    } else {
+      hi = mid - 1;
+      above = c;
+    }
   }
-  int r = i - count(lo + 1);
+  int r = i - above;
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
     const bool has = lo >= base[c] && lo < base[c] + n[c];
@@ -352,15 +367,21 @@ __device__ __forceinline__ UnitAt unit_search(const int32_t* cu, const int32_t* 
 
 __device__ __forceinline__ UnitAt unit_by_work(const int32_t* cu, const int32_t* ctx_lens, int num_seqs, int UR,
                                                int i, int cols) {
-  if (num_seqs <= 64) return unit_search<1>(cu, ctx_lens, num_seqs, UR, i, cols);
-  if (num_seqs <= kUnitSeqs) return unit_search<kUnitChunks>(cu, ctx_lens, num_seqs, UR, i, cols);
+  if (num_seqs > 1 && num_seqs <= 64) return unit_search<1>(cu, ctx_lens, num_seqs, UR, i, cols);
+  if (num_seqs > 1 && num_seqs <= kUnitSeqs) {
+    return unit_search<kUnitChunks>(cu, ctx_lens, num_seqs, UR, i, cols);
+  }
+  if (num_seqs == 1 && i >= cols && i < 2 * cols) i = 3 * cols - 1 - i;
   UnitAt u{-1, 0, 0, 0, 0, 0};
   const int s = i % num_seqs, rank = i / num_seqs;
   u.row0 = cu[s];
   u.rows = cu[s + 1] - u.row0;
   u.ctx = ctx_lens[s];
-  u.unit = (max(u.rows, 0) + UR - 1) / UR - 1 - rank;
+  const int n = (max(u.rows, 0) + UR - 1) / UR;
+  u.unit = n - 1 - rank;
   if (u.unit >= 0) u.seq = s;
+  u.end = s + num_seqs * n;  // (of this sequence; the caller's steps keep to it)
+  if (num_seqs == 1 && n > cols) u.end = max(n, 2 * cols);
   return u;
 }
 
@@ -586,8 +607,8 @@ __global__ __launch_bounds__(kPThreads, DIRECT ? 2 : pf_wg_per_cu<D>()) void pre
     }
     if constexpr (DIRECT) {
       const UnitAt at = unit_by_work(cu_seqlens, context_lens, a.num_seqs, UR, u, 0);
-      // The next item and their number wait in LDS, not in scalar registers (at their limit).
-      sched_next[w] = make_int2(u + (int)(gridDim.x / ngroups), at.total);
+      // The next item and their end wait in LDS, not in scalar registers (at their limit).
+      sched_next[w] = make_int2(u + (int)(gridDim.x / ngroups), at.end);
       if (at.seq < 0) return false;
       un.s = at.seq;
       un.row0 = at.row0;
@@ -1488,6 +1509,7 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
               make_float4(o[b][4 * j] * inv, o[b][4 * j + 1] * inv, o[b][4 * j + 2] * inv, o[b][4 * j + 3] * inv);
         }
     }
+    if (i + (int)gridDim.y >= at.end) break;
     __syncthreads();  // every wave is done with the LDS tiles before the next unit's copies
   }
 }
@@ -1639,7 +1661,9 @@ extern "C" int rg_prefill_packed(const void* query, const void* key_cache, const
     const int64_t qmax = std::min<int64_t>(std::max<int32_t>(max_query_len, 1), num_tokens);
     const int64_t groups = num_heads / GW, cus = device_cu_count();
     if (cus % groups == 0 && head_dim <= 128) a.sched_cols = (int32_t)(cus / groups);  // (256: one workgroup per CU)
-    const int64_t units = (qmax + UR - 1) / UR, items = units * num_seqs, cols = std::max(a.sched_cols, 1);
+    // Units: at most those of the longest sequence in every sequence, and no more than the tokens give.
+    const int64_t units = (qmax + UR - 1) / UR, cols = std::max(a.sched_cols, 1);
+    const int64_t items = std::min(units * num_seqs, (num_tokens + num_seqs * (UR - 1)) / UR);
     // Past kUnitSeqs a workgroup keeps to one sequence (unit_by_work): a multiple of num_seqs.
     const int64_t wgs = num_seqs > kUnitSeqs
                             ? num_seqs * std::max<int64_t>(1, std::min<int64_t>(units, 65535 / num_seqs))

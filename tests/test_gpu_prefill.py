@@ -254,6 +254,18 @@ def test_prefill_f32_units_by_work(device, kernels, nseq, H, Hkv, D, max_query_l
     _run(device, kernels, w, seed=nseq + 1, max_query_len=max_query_len)
 
 
+@pytest.mark.parametrize("max_query_len", [None, 1])
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("lens,H,Hkv", [([1100], 32, 8), ([2100], 32, 8), ([33], 24, 8), ([700] + [1] * 63, 32, 8),
+                                        ([1] * 100 + [600] + [3] * 50, 8, 2), ([5] * 290 + [300], 8, 2)])
+def test_prefill_one_long_sequence(device, kernels, lens, H, Hkv, dt, max_query_len):
+    """One sequence (its units between one and two per column, past two, a single one) and one long
+    sequence among short ones in every form of the deal: workgroups stop at the last unit that exists,
+    and the fp32 grid is bounded by the tokens."""
+    w = _gqa_workload(H // Hkv, 64, lens, [0] * len(lens), seed=len(lens), dt=dt, H=H)
+    _run(device, kernels, w, seed=len(lens) + H, max_query_len=max_query_len, row_sample=True)
+
+
 def _run_f32_rows(device, kernels, D, q0, key0, val):
     """One sequence of len(key0) rows at 4 / 1 heads: q row r is q0[r] and key t key0[t] in their first
     dim (0 in the others), value t is val[t] in every dim; scale 1.  Returns the first head's dims."""
