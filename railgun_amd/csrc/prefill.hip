@@ -1264,20 +1264,22 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
 
     // Copy i of wave w moves LDS pieces 64 (w PER + i) + lane of an operand's tile; keys past the
     // unit's last read the last one (masked below).  Lane l holds the cache offset of key l % 32
-    // of a tile: its block number is loaded two iterations before its K copy (table_entry) and
-    // turned into the offset (row_offset) when that copy goes out, so that no copy waits for a
-    // table read; the V copies fetch the offsets of their rows from those lanes.
+    // of a tile: its block number is loaded two iterations before its K copy (table_entry; those of
+    // the first three tiles at once, before the q rows) and turned into the offset (row_offset) when
+    // that copy goes out, so that no copy waits for a table read; the V copies fetch the offsets of
+    // their rows from those lanes.
     const int kl = lane & 31;
-    int blk = 0, in_blk = 0;
+    struct Entry { int blk, in_blk; };
     auto table_entry = [&](int kt) __attribute__((always_inline)) {
-      const int kk = min(kt * kPT + kl, nkeys - 1);
+      const int kk = max(min(kt * kPT + kl, nkeys - 1), 0);
       const int b = kk / bs;
-      in_blk = kk - b * bs;
-      blk = bt[b];
+      return Entry{bt[b], kk - b * bs};
     };
-    auto row_offset = [&]() __attribute__((always_inline)) {
-      return (int64_t)blk * a.kv_stride + ((int64_t)kvh * bs + in_blk) * D;
+    auto row_offset = [&](Entry e) __attribute__((always_inline)) {
+      return (int64_t)e.blk * a.kv_stride + ((int64_t)kvh * bs + e.in_blk) * D;
     };
+    const Entry e0 = table_entry(0), e1 = table_entry(1);
+    Entry ahead = table_entry(2);
     auto issue_k = [&](int kt, int64_t roff) __attribute__((always_inline)) {
       const uint32_t off = (uint32_t)((kt & 1) * TILE * 4);
 #pragma unroll
@@ -1444,26 +1446,23 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
     // softmax of tile kt: a wave alone on its SIMD then keeps the matrix core busy through the
     // softmax.
     if (ntiles > 0) {
-      int64_t roff1;
-      table_entry(0);
-      {
-        const int64_t roff0 = row_offset();
-        table_entry(1);
-        issue_k(0, roff0);
-        issue_v(0, roff0);
-      }
-      roff1 = row_offset();
-      table_entry(2);
+      const int64_t roff0 = row_offset(e0);
+      int64_t roff1 = row_offset(e1);
+      asm volatile("" ::"v"(roff0), "v"(roff1));  // formed before the copies: a later wait would be for those too
+      issue_k(0, roff0);
+      issue_v(0, roff0);
       if (ntiles > 1) issue_k(1, roff1);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      // K(0) is there: only V(0) and K(1) have been sent out after it.
+      if (ntiles > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
       tile_barrier();
       f32x16 st = f32x16{};
       if (kfull > 0) st = scores(0, [](auto) {});
       auto copies = [&](int kt) __attribute__((always_inline)) {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // this wave's copies (and LDS reads)
         tile_barrier();                                              // ... and every wave's
-        const int64_t roff2 = row_offset();
-        table_entry(kt + 3);
+        const int64_t roff2 = row_offset(ahead);
+        ahead = table_entry(kt + 3);
         if (kt + 2 < ntiles) issue_k(kt + 2, roff2);
         if (kt + 1 < ntiles) issue_v(kt + 1, roff1);
         roff1 = roff2;
