@@ -1662,16 +1662,27 @@ extern "C" int rg_prefill_packed(const void* query, const void* key_cache, const
     if (cus % groups == 0 && head_dim <= 128) a.sched_cols = (int32_t)(cus / groups);  // (256: one workgroup per CU)
     // Units: at most those of the longest sequence in every sequence, and no more than the tokens give.
     const int64_t units = (qmax + UR - 1) / UR, cols = std::max(a.sched_cols, 1);
-    const int64_t items = std::min(units * num_seqs, (num_tokens + num_seqs * (UR - 1)) / UR);
     // Past kUnitSeqs a workgroup keeps to one sequence (unit_by_work): a multiple of num_seqs.
-    const int64_t wgs = num_seqs > kUnitSeqs
-                            ? num_seqs * std::max<int64_t>(1, std::min<int64_t>(units, 65535 / num_seqs))
-                            : std::min<int64_t>(ceil_div(items, cols) * cols, 65535);
-    const dim3 grid((unsigned)groups, (unsigned)wgs);
+    auto wgs = [&](int64_t seqs) {
+      const int64_t items = std::min(units * seqs, (num_tokens + seqs * (UR - 1)) / UR);
+      return seqs > kUnitSeqs ? seqs * std::max<int64_t>(1, std::min<int64_t>(units, 65535 / seqs))
+                              : std::min<int64_t>(ceil_div(items, cols) * cols, 65535);
+    };
+    // Its item index, below sequences x 2 (units + 1), has 32 bits: one launch holds all but absurd
+    // batches (65,535 sequences with more than 500,000 rows), the rest go in ranges of sequences.
+    const int64_t most = std::max<int64_t>(kUnitSeqs, INT32_MAX / (2 * (num_tokens / UR + 2)));
     auto go = [&](auto dtag, auto gtag) {
       constexpr int D = decltype(dtag)::value;
       constexpr int W = decltype(gtag)::value;
-      hipLaunchKernelGGL((prefill_f32_kernel<D, W>), grid, dim3(kPThreads), 0, s, a);
+      for (int64_t s0 = 0; s0 < num_seqs; s0 += most) {
+        PrefillArgs part = a;
+        part.num_seqs = (int32_t)std::min<int64_t>(most, num_seqs - s0);
+        part.block_table += s0 * max_blocks_per_seq;
+        part.context_lens += s0;
+        part.cu_seqlens += s0;
+        const dim3 grid((unsigned)groups, (unsigned)wgs(part.num_seqs));
+        hipLaunchKernelGGL((prefill_f32_kernel<D, W>), grid, dim3(kPThreads), 0, s, part);
+      }
     };
     auto go_gw = [&](auto dtag) {
       if (GW == 4) go(dtag, std::integral_constant<int, 4>{});
