@@ -213,7 +213,8 @@ int rg_silu_and_mul_interleaved(const void* gate_up, void* out, int32_t num_rows
  * 128, x and weight rows 16-byte aligned, out rows 8-byte aligned; RG_ERR_NOT_SUPPORTED
  * otherwise (larger batches belong to a library GEMM).  A workspace of
  * rg_linear_workspace_bytes (16-byte aligned) lets narrow or deep layers split K over more
- * workgroups; without it (NULL, or smaller) the call runs unsplit.  New entry: the reference
+ * workgroups; a smaller one as far as it holds the partials, without one (NULL) or with an
+ * unaligned one the call runs unsplit.  New entry: the reference
  * runs these projections through candle's cuBLAS GEMMs. */
 int rg_linear(const void* x, const void* weight, void* out, int32_t num_rows,
               int32_t out_features, int32_t in_features, int64_t x_row_stride,

@@ -164,6 +164,26 @@ def test_linear_splits_long_walks(device, M, N, K, dt):
     assert torch.equal(res, (r.float() + out.float()).to(TORCH[dt])), "the residual add of the rounded sum"
 
 
+@pytest.mark.parametrize("M,N,K", [(64, 4096, 14336), (16, 3072, 8192), (33, 2048, 8192), (1, 4096, 4096)])
+@pytest.mark.parametrize("part", [0.0, 0.5, 0.75])
+def test_linear_smaller_workspace(device, M, N, K, part):
+    """A workspace that does not hold the best plan's partials: the call takes a plan with fewer splits,
+    writes nothing past the bytes it was given, and gives the same product."""
+    nbytes = linear_workspace_bytes(M, N, K)
+    assert nbytes > 0, "split on a 256-CU device"
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=device).to(torch.bfloat16)
+    w = (0.02 * torch.randn(N, K, generator=g, device=device)).to(torch.bfloat16)
+    r = torch.randn(M, N, generator=g, device=device).to(torch.bfloat16)
+    given = int(nbytes * part) // 16 * 16
+    ws = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=device)
+    out = linear(x, w, workspace=ws[:given])
+    res = linear_residual(x, w, r.clone(), ws[:given])
+    _check(out, x, w, f"{M}x{N}x{K} {part}", ref_on_device=True)
+    assert torch.equal(res, (r.float() + out.float()).to(torch.bfloat16)), "the residual add of the rounded sum"
+    assert bool((ws[given:] == 0xA5).all())
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("M,I,K", [(128, 8192, 2048), (1, 8192, 2048), (37, 512, 256), (100, 1040, 1024)])
 def test_linear_silu_mul(device, M, I, K, dt):
