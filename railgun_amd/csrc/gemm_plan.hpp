@@ -44,14 +44,15 @@ inline int ring_bytes(int nb, int mb, int reserve = 0) {
 //            (0.047 us per 16 rows x 128 k: 4 KB of copies),
 //   turn = 3 us + 0.18 us x sqrt(2 / chunks in flight) x chunks / S: a workgroup walks its chunks one
 //          after the other, a copy's round trip over the chunks in flight each, however few bytes
-//          they hold (4096 x 14336 unsplit, 112 chunks in turn, took 30 us whatever its rows),
+//          they hold (4096 x 14336 unsplit, 112 chunks in turn, took 30 us at 1 and at 16 rows alike),
 //   serial = max(stream, ceil(workgroups / R) x turn), weights = N K 2 B / 5.5 TB/s,
 //   time = max(serial, weights) + 0.2 min(serial, weights) + 0.1 stream + (S > 1: 2 us + S M N 8 B /
 //          3 TB/s for the partials and their reduce).
-// Without the turn the model left deep layers unsplit: 4096 x 14336 at 1 / 27 / 64 rows 30.5 / 33.2
-// / 36.7 us against 22.1 / 22.9 / 31.8 now (the weights alone 18.9 at 6.2 TB/s), 3072 x 8192 at 1
-// to 16 rows 17.8 against 13.5.  Over that sweep its pick is 1.6 % from the measured best on average
-// (7.9 % without) and nowhere slower than before.
+// Without the turn the model left deep layers unsplit: 4096 x 14336 at 1 / 27 / 64 rows 30.3 / 32.7
+// / 35.9 us against 21.9 / 22.9 / 27.3 now (the weights alone 18.9 at 6.2 TB/s), 3072 x 8192 at 1
+// to 16 rows 17.4 against 13.6; of 182 shapes one is slower than without it, by 2 % (3072 x 3072 at 8
+// rows).  The pick is 2.4 % from the best of all plans on average, 21 % at worst (2048 x 8192 at 33
+// rows; profiles/skinny_gemm_plan_sweep.txt).
 // Each workgroup streams its rows of X and its columns of W once per K range; small row tiles
 // cut the X bytes of narrow layers, and the XCD-aware order keeps their re-reads of W in L2.
 struct GemmPlan { int nb, mb, mtiles, splits, xcd; };

@@ -1188,9 +1188,9 @@ __global__ __launch_bounds__(kPThreads, DIRECT ? 2 : pf_wg_per_cu<D>()) void pre
 // the head group as the fastest dimension a multiple of 8 groups keeps each kv-head's K/V on one
 // die.  Measured (kernel and cache write, us a call): 12 prompts of 128 to 2,048 tokens at head_dim
 // 128 1,749 with every sequence's units from its end, one sequence after the other, 1,370 sorted;
-// 16 prompts of 40 to 512 behind up to 1,000 cached at head_dim 64 390 -> 317; the 5 prompts below
-// 122.4 -> 114.6; one prompt of 40 rows the same (15.6).  The reversed second deal of unit_by_work
-// is the last 3 us of the 114.6, and 51.2 -> 46.2 for 3 prompts of 300 to 512.
+// 16 prompts of 40 to 512 behind up to 1,000 cached at head_dim 64 390 -> 317; 5 prompts of 171 to
+// 964 rows at 32 / 8 heads of 64 122.4 -> 114.6; one prompt of 40 rows the same.  The reversed second
+// deal of unit_by_work is the last 3 us of the 114.6, and 51.2 -> 46.2 for 3 prompts of 300 to 512.
 //
 //  * Bound: the fp32 MFMAs, 64 cycles each, 2 x D / 2 of them per tile.  The 32-key K and V tiles
 //    reach LDS by direct global -> LDS copies into two buffers each, K a tile further ahead than
@@ -1198,7 +1198,7 @@ __global__ __launch_bounds__(kPThreads, DIRECT ? 2 : pf_wg_per_cu<D>()) void pre
 //    them, both operands read from LDS a few steps ahead of their MFMA, so that a wave keeps its
 //    SIMD's matrix core busy by itself: the last units of a call run one or two to a CU.  Without
 //    that (QK, softmax, PV in turn, operands read as they were used, a table read in front of
-//    every copy) the 5 prompts above took 146 us, 113 with it (75 TFLOP/s, 49 % of what a large
+//    every copy) the kernel took 146 us for those 5 prompts, 113 with it (75 TFLOP/s, 49 % of what a large
 //    fp32 product reaches here); 12 prompts of 128 to 2,048 tokens at head_dim 128 2,158 -> 1,749
 //    us a call with the cache write, 6 of up to 700 behind up to 500 cached at head_dim 256 529 ->
 //    304.  The arithmetic and its order are those of softmax and PV in turn; new_maximum below says
@@ -1368,10 +1368,10 @@ __global__ __launch_bounds__(kPThreads, D > 128 ? 1 : 2) void prefill_f32_kernel
     // scores, in the parts 0 .. 7 that ride along with the next tile's QK steps; rescale then applies
     // the new maximum to o.
     // v_exp_f32 by itself has no subnormal results, and exp2f, which has, in its place costs 7 % of the
-    // call at head_dim 64 and 4 % at 128 (fp32 MFMAs leave the vector units no free cycles).  So the
-    // parts take the instruction, and a tile with a factor or a probability below 2^-126 (`deep`, seen
-    // by its smallest score) is done before them with exp2f, which costs 1.3 % and 0.6 %.  A row whose
-    // scores are NaN gives NaN.
+    // call at head_dim 64 and 4 % at 128, spread over the MFMAs or not.  So the parts take the
+    // instruction, and a tile with a factor or a probability below 2^-126 (`deep`, seen by its smallest
+    // score) is done before them with exp2f, which costs 1.3 % and 0.6 %.  A row whose scores are NaN
+    // gives NaN.
     float mref = 0.f, alpha = 0.f, ps = 0.f;
     bool deep = false;
     auto new_maximum = [&](const f32x16& st) __attribute__((always_inline)) {

@@ -228,7 +228,7 @@ class RailgunLlama:
         self.mlp_choice: dict = {}
         # The fused MLP form reads the gate/up weight with its rows interleaved in blocks of 16:
         # each layer's weight is replaced by that layout in place (one copy held, not two); the
-        # separate form then de-interleaves the projection's output columns instead.
+        # separate form reads the projection's columns in that order (rg_silu_and_mul_interleaved).
         self._w_gate_up_il: dict = {}  # layer -> interleaved copy, only for weights left stacked
         if mode != "blas" and self.dtype in (torch.bfloat16, torch.float16) and cfg.intermediate_size % 16 == 0:
             for L in weights.layers:

@@ -227,8 +227,7 @@ def test_interleave_gate_up_layout():
 def test_deinterleave_gate_up_inverts_the_layout():
     """deinterleave_gate_up undoes interleave_gate_up on the weight rows, and on the columns of
     a product: x @ interleaved^T, de-interleaved, is x @ w_gate_up^T exactly (a permutation of
-    the same sums), which is what the model's separate MLP form relies on once the weight is
-    held interleaved."""
+    the same sums), which the test of rg_silu_and_mul_interleaved compares against."""
     import torch
 
     from railgun_amd.ops import deinterleave_gate_up, interleave_gate_up
