@@ -1998,10 +1998,14 @@ size_t stream_bytes(const Shape& sh, int32_t workers, StreamScratch* carve, void
 //   Up to two per CU: 64 tokens, 0.92 at worst (264 to 512 segments); at 128 already 1.33, at 320
 // 1.48.  More: never (1,024 segments of 64 tokens 1.27 to 1.60).
 bool short_applies(const Shape& sh, int elem_bytes) {
-  const int64_t tokens = (int64_t)sh.MB * sh.bs, segments = (int64_t)sh.B * sh.Hkv, cus = device_cu_count();
+  const int64_t tokens = (int64_t)sh.MB * sh.bs, segments = (int64_t)sh.B * sh.Hkv;
   const int64_t widest = (sh.D == 64 ? 224 : 160) + (elem_bytes == 4 ? 32 : 0);  // KB of K and V
-  return (sh.D == 64 || sh.D == 128) && sh.H / sh.Hkv <= 8 && tokens <= kShortMaxTokens && sh.B <= 65535 &&
-         (segments <= cus ? tokens * sh.D * 2 * elem_bytes <= widest << 10 : segments <= 2 * cus && tokens <= 64);
+  if ((sh.D != 64 && sh.D != 128) || sh.H / sh.Hkv > 8 || tokens > kShortMaxTokens || sh.B > 65535 ||
+      tokens * sh.D * 2 * elem_bytes > widest << 10) {
+    return false;
+  }
+  const int64_t cus = device_cu_count();  // (two calls of the runtime: asked for small tables only)
+  return segments <= cus || (segments <= 2 * cus && tokens <= 64);
 }
 
 template <typename T, int D, int G, bool ROPE = false>
